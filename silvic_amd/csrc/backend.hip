@@ -395,15 +395,14 @@ struct Context {
     DevBuf<FeatDev> dfeats;
     DevBuf<ColGroup> d_cgs;
     DevBuf<uint32_t> d_fmt;  // per slab and k_step_rows workgroup: the format of its partial (1 packed, 0 pairs)
-    DevBuf<int32_t> unit_feat;   // k_step_scan's units: UNIT_FEATS numerical features each, -1 padding
+    DevBuf<UnitRec> unit_recs;   // k_step_children's scan units: UNIT_FEATS features each, -1 padding
     DevBuf<uint32_t> unit_segl;  // and their lanes a feature (64, 16, 4)
-    DevBuf<uint32_t> cat_feats;  // the categorical features of the slabs
-    uint32_t ncat = 0;
-    uint32_t ncg = 0;  // column groups of k_step_reduce
-    uint32_t nsg = 0;  // scan units of k_step_scan
-    bool has_seg_units = false;  // some units scan several features (k_step_scan_seg)
-    uint32_t nseg_units = 0;     // those units, first in the unit list
-    bool has_narrow64 = false;   // some units scan one byte feature (k_step_scan<false>)
+    DevBuf<int32_t> wide_feats;  // the two-byte features (k_step_scan)
+    uint32_t ncgb = 0;  // column groups of byte slabs (k_step_children)
+    uint32_t ncgw = 0;  // column groups of two-byte slabs (k_step_reduce), after those
+    uint32_t nwide = 0;
+    bool has_seg_units = false;  // some units scan several features a wave
+    bool has_cat = false;        // some units scan a categorical feature
     uint64_t step_partial_pairs = 0;
     uint32_t part_len = 0;
     std::vector<uint8_t> used;
@@ -978,8 +977,8 @@ struct Context {
         return false;
     }
 
-    // The slab tables: per slab slot its feature's flat bins, the column groups of k_step_reduce, the numerical
-    // features (in groups of CG_COLS) of k_step_scan, the categorical ones of k_step_cat, and the partial buffers.
+    // The slab tables: per slab slot its feature's flat bins, the column groups and scan units of k_step_children, the
+    // column groups of k_step_reduce and the features of k_step_scan (two-byte slabs), and the partial buffers.
     void build_slab_tables() {
         partial.alloc(static_cast<size_t>(hist_cap) * 256 * max_width * 2);
         std::vector<uint32_t> all_bins;  // slab_col_bins
@@ -1027,22 +1026,34 @@ struct Context {
             hip_check(hipMemcpy(slab_pos_word.p, all_pos.data(), all_pos.size() * 4, hipMemcpyHostToDevice), "upload dense slab");
             hip_check(hipMemcpy(slab_slot_flat.p, all_slot.data(), all_slot.size() * 4, hipMemcpyHostToDevice), "upload dense slab");
         }
-        // groups of CG_COLS slab columns for k_step_reduce, the numerical features in groups of CG_COLS for
-        // k_step_scan, and the categorical ones for k_step_cat
+        // groups of CG_COLS slab columns, the byte slabs' first with their scan units (k_step_children), then the
+        // two-byte slabs' (k_step_reduce) and their features (k_step_scan)
         {
             std::vector<ColGroup> cg;
-            std::vector<int32_t> sfeat;
-            std::vector<uint32_t> cats;
+            std::vector<UnitRec> recs;
+            std::vector<uint32_t> usegl;
+            std::vector<int32_t> wfeats;
             uint64_t poff = 0;
+            ncgb = ncgw = 0;
+            has_seg_units = has_cat = false;
             for (size_t si = 0; si < slabs.size(); ++si) {
                 Slab &s = slabs[si];
                 s.step_partial_off = poff;
                 // a wide slab's virtual column v holds bins q, q + 4, ... (q = v / (W/4)) of feature v % (W/4); a
-                // packed slab's column c holds feature seg * W + c in bins [seg, seg + 1) * 2^seg_shift
+                // packed slab's column c holds feature seg * W + c in bins [seg, seg + 1) * 2^seg_shift; a dense slab's
+                // byte p is column p % 128, at the LDS row of its word
                 const uint32_t cap = s.capacity();
+                std::vector<std::vector<std::pair<uint32_t, uint32_t>>> held(s.width / CG_COLS);  // (feature, LDS row)
+                if (!s.wide)
+                    for (uint32_t i = 0; i < nt_feat.size(); ++i) {
+                        if (nt_slab[i] != si) continue;
+                        const uint32_t at = nt_slab_col[i], col = at % s.width;
+                        const uint32_t row = s.dense_passes ? s.pos_word[at] / s.width : (at / s.width) << s.seg_shift();
+                        held[col / CG_COLS].emplace_back(nt_feat[i], 256u * (col % CG_COLS) + row);
+                    }
                 for (uint32_t c0 = 0; c0 < s.width; c0 += CG_COLS) {
                     ColGroup x{poff, s.width, c0, static_cast<uint32_t>(si) * k1_groups(), {}, {}, {}, s.seg_shift(),
-                               s.dense_passes ? 1u : 0u, static_cast<uint32_t>(s.slot_off)};
+                               s.dense_passes ? 1u : 0u, static_cast<uint32_t>(s.slot_off), s.q32 ? 1u : 0u, 0u, 0u};
                     for (uint32_t k = 0; k < CG_COLS && !s.dense_passes; ++k) {
                         const uint32_t v = c0 + k;
                         x.stride[k] = s.wide ? 4u : 1u;
@@ -1054,64 +1065,72 @@ struct Context {
                             x.bins[seg][k] = real && m.num_bins > q ? (m.num_bins - q + (s.wide ? 3 : 0)) / (s.wide ? 4 : 1) : 0u;
                         }
                     }
+                    if (s.wide) {
+                        cg.push_back(x);
+                        ++ncgw;
+                        continue;
+                    }
+                    // the group's scan units: a feature a wave while the block's eight waves take both children of each
+                    // at once (up to four features); beyond, numerical features of at most 16 bins 16 a wave and of at
+                    // most 64 bins 4 a wave
+                    const auto &fs = held[c0 / CG_COLS];
+                    if (fs.empty()) continue;  // padding columns: nothing reads their histogram
+                    x.unit_first = static_cast<uint32_t>(usegl.size());
+                    const bool segmented = fs.size() > CG_COLS;
+                    for (uint32_t segl : {64u, 16u, 4u}) {
+                        std::vector<std::pair<uint32_t, uint32_t>> members;
+                        for (const auto &f : fs) {
+                            const srocm_feature &m = feats[f.first];
+                            const bool one = !segmented || m.kind == SROCM_BINS_CATEGORICAL || m.num_bins > 64;
+                            if ((one ? 64u : (m.num_bins > 16 ? 16u : 4u)) == segl) members.push_back(f);
+                            has_cat = has_cat || m.kind == SROCM_BINS_CATEGORICAL;
+                        }
+                        const size_t per = 64 / segl;
+                        for (size_t b = 0; b < members.size(); b += per) {
+                            for (size_t k = 0; k < UNIT_FEATS; ++k) {
+                                UnitRec r{-1, 0u, FeatDev{}};
+                                if (k < per && b + k < members.size()) {
+                                    const uint32_t f = members[b + k].first;
+                                    const srocm_feature &m = feats[f];
+                                    r = UnitRec{static_cast<int32_t>(f), members[b + k].second,
+                                                FeatDev{m.num_bins, m.hist_offset, m.kind, m.nan_bin,
+                                                        static_cast<uint32_t>(std::max(feat_nt[f], 0)), 0u}};
+                                }
+                                recs.push_back(r);
+                            }
+                            usegl.push_back(segl);
+                            has_seg_units = has_seg_units || segl != 64;
+                        }
+                    }
+                    x.unit_count = static_cast<uint32_t>(usegl.size()) - x.unit_first;
                     cg.push_back(x);
+                    ++ncgb;
                 }
-                for (uint32_t f : s.feats) {
-                    if (feats[f].kind == SROCM_BINS_CATEGORICAL) cats.push_back(f);
-                    else sfeat.push_back(static_cast<int32_t>(f));
-                }
+                if (s.wide)
+                    for (uint32_t f : s.feats) wfeats.push_back(static_cast<int32_t>(f));
                 poff += static_cast<uint64_t>(k1_groups()) * step_partial_stride(s.width);
             }
-            // scan units: byte features of at most 16 bins 16 a wave, of at most 64 bins 4 a wave, the others (and
-            // two-byte features) one a wave; when that saves under a quarter of the waves, every feature one a wave
-            // (the units of several features take a kernel of their own)
-            auto unit_lanes = [&](int32_t f) {
-                const uint32_t nb = feats[f].num_bins;
-                return group_bits[feats[f].group] == 16 || nb > 64 ? 64u : (nb > 16 ? 16u : 4u);
-            };
-            size_t seg_units = 0;
-            for (uint32_t segl : {4u, 16u, 64u}) {
-                size_t n = 0;
-                for (int32_t f : sfeat) n += unit_lanes(f) == segl;
-                seg_units += (n + 64 / segl - 1) / (64 / segl);
-            }
-            const bool segmented = seg_units * 4 <= sfeat.size() * 3;
-            std::vector<int32_t> ufeat;
-            std::vector<uint32_t> usegl;
-            for (uint32_t segl : {4u, 16u, 64u}) {
-                std::vector<int32_t> members;
-                for (int32_t f : sfeat)
-                    if ((segmented ? unit_lanes(f) : 64u) == segl) members.push_back(f);
-                const size_t per = 64 / segl;
-                for (size_t b = 0; b < members.size(); b += per) {
-                    for (size_t k = 0; k < UNIT_FEATS; ++k)
-                        ufeat.push_back(k < per && b + k < members.size() ? members[b + k] : -1);
-                    usegl.push_back(segl);
-                }
-            }
+            nwide = static_cast<uint32_t>(wfeats.size());
             d_fmt.alloc(std::max<size_t>(slabs.size(), 1) * k1_groups());
-            ncg = static_cast<uint32_t>(cg.size());
-            nsg = static_cast<uint32_t>(usegl.size());
-            has_seg_units = segmented;
-            nseg_units = 0;
-            while (nseg_units < usegl.size() && usegl[nseg_units] != 64) ++nseg_units;
-            has_narrow64 = false;
-            for (size_t u = 0; u < usegl.size(); ++u)
-                if (usegl[u] == 64 && group_bits[feats[ufeat[u * UNIT_FEATS]].group] != 16) has_narrow64 = true;
             step_partial_pairs = std::max<uint64_t>(poff, 1);
             d_cgs.alloc(std::max<size_t>(cg.size(), 1));
-            unit_feat.alloc(std::max<size_t>(ufeat.size(), 1));
+            if (!has_seg_units) {  // a feature a unit: CG_COLS records a group, found by the group's index alone
+                std::vector<UnitRec> flat(static_cast<size_t>(ncgb) * CG_COLS, UnitRec{-1, 0u, FeatDev{}});
+                for (uint32_t k = 0; k < ncgb; ++k)
+                    for (uint32_t u = 0; u < cg[k].unit_count; ++u) flat[CG_COLS * k + u] = recs[static_cast<size_t>(cg[k].unit_first + u) * UNIT_FEATS];
+                recs = std::move(flat);
+            }
+            unit_recs.alloc(std::max<size_t>(recs.size(), 1));
             unit_segl.alloc(std::max<size_t>(usegl.size(), 1));
+            wide_feats.alloc(std::max<size_t>(wfeats.size(), 1));
             if (!cg.empty())
                 hip_check(hipMemcpy(d_cgs.p, cg.data(), cg.size() * sizeof(ColGroup), hipMemcpyHostToDevice), "upload column groups");
-            if (!ufeat.empty()) {
-                hip_check(hipMemcpy(unit_feat.p, ufeat.data(), ufeat.size() * 4, hipMemcpyHostToDevice), "upload scan units");
+            if (!usegl.empty()) {
+                hip_check(hipMemcpy(unit_recs.p, recs.data(), recs.size() * sizeof(UnitRec), hipMemcpyHostToDevice), "upload scan units");
                 hip_check(hipMemcpy(unit_segl.p, usegl.data(), usegl.size() * 4, hipMemcpyHostToDevice), "upload scan units");
             }
-            ncat = static_cast<uint32_t>(cats.size());
-            cat_feats.alloc(std::max<size_t>(cats.size(), 1));
-            if (!cats.empty())
-                hip_check(hipMemcpy(cat_feats.p, cats.data(), cats.size() * 4, hipMemcpyHostToDevice), "upload categorical features");
+            if (!wfeats.empty())
+                hip_check(hipMemcpy(wide_feats.p, wfeats.data(), wfeats.size() * 4, hipMemcpyHostToDevice), "upload two-byte features");
         }
     }
 
@@ -1148,7 +1167,10 @@ struct Context {
         step_target = st;
         if (!relayout) {
             build_slab_tables();
-            if (grow_capacity) step_partial.alloc(2 * step_partial_pairs);
+            if (grow_capacity) {
+                step_partial.alloc(2 * step_partial_pairs);
+                alloc_cands();
+            }
             sync();
             return;
         }
@@ -1161,7 +1183,10 @@ struct Context {
             repack(train.col.p + static_cast<size_t>(nt) * rows * cb, static_cast<uint32_t>(cb), 0, col16 ? 16u : 8u, rows, to);
         }
         build_slab_tables();
-        if (grow_capacity) step_partial.alloc(2 * step_partial_pairs);
+        if (grow_capacity) {
+            step_partial.alloc(2 * step_partial_pairs);
+            alloc_cands();
+        }
         sync();
     }
 
@@ -1958,15 +1983,19 @@ struct Context {
     DevBuf<uint8_t> d_splittable, d_eval, d_mask;
     std::vector<uint8_t> d_mask_host;  // what d_mask holds (empty: unknown), so an unchanged mask is not uploaded again
     DevBuf<ScanJob> d_jobs;
-    DevBuf<FeatCand> d_cands;
+    DevBuf<FeatCand> d_root_cands, d_cands;
+    DevBuf<double> d_cand_gain;
+    DevBuf<int32_t> d_cand_feat;
     DevBuf<RowRun> d_runs;            // end of a tree: runs of rows to bring into ascending order
     DevBuf<MergeJob> d_merges;        // end of a tree: leaves whose expansion was dropped
     DevBuf<uint32_t> d_starts;
     Pinned<uint8_t> h_fix;            // staging of the runs and merges (rewritten only after a sync)
-    // split steps (k_step_rows, k_step_reduce, k_step_scan, k_step_cat, k_step_select)
+    // split steps (k_step_rows, k_step_children, k_step_reduce, k_step_scan, k_step_select)
     DevBuf<int32_t> step_partial;            // per slab: [cus + JMAX][256 * W] {g, h}
     DevBuf<unsigned long long> tile_status;  // per partition tile
     DevBuf<uint32_t> fin_counts;             // the jobs-selected counter of k_step_select
+    DevBuf<int64_t> child_scratch;           // k_step_children: the sums of shared jobs' shares, and their arrivals
+    DevBuf<uint32_t> child_counts;
     uint64_t epochs_used = 0;
     uint32_t last_steps = 0;                 // split steps of the last tree (the first guess for the next)
     // The control block, the tree arrays, the leaves' row ranges and the committed leaves' speculative leaves, in one
@@ -1989,6 +2018,11 @@ struct Context {
     uint32_t grow_capacity = 0;
 
     uint32_t k1_groups() const { return step_target + JMAX; }  // k_step_rows' grid
+    // The records a step's jobs take in its plan at most (ceil(g / CHILD_SHARE) - 1 <= g / CHILD_SHARE besides one each),
+    // and the scratch rows of jobs of several shares (fewer than k1 / CHILD_SPLIT of them).
+    uint32_t child_shares(uint32_t jcap) const { return std::min<uint32_t>(CHILD_MAX, jcap + k1_groups() / CHILD_SHARE); }
+    uint32_t child_rows() const { return std::min<uint32_t>(CHILD_MAX, k1_groups() / CHILD_SHARE + k1_groups() / CHILD_SPLIT + 1); }
+    uint32_t nslot() const { return std::max<uint32_t>(ncgb + nwide, 1); }
     uint32_t scan_blocks() const { return 8 * cus; }   // k_step_scan's grid: four waves a block, a wave per item
     uint32_t reduce_blocks() const { return 8 * cus; } // k_step_reduce's grid
 
@@ -2005,7 +2039,8 @@ struct Context {
         d_mask.alloc(nf);
         d_mask_host.clear();
         d_jobs.alloc(1);
-        d_cands.alloc(static_cast<size_t>(JMAX) * 2 * nf);
+        d_root_cands.alloc(nf);
+        alloc_cands();
         tree_layout = TreeLayout(L);
         dtree.alloc(tree_layout.bytes);
         // host staging at its largest, so that no tree allocates pinned memory
@@ -2022,6 +2057,17 @@ struct Context {
         fin_counts.alloc(1);
         reset_step_state();
         grow_capacity = L;
+    }
+
+    // The candidate slots and the shares' scratch follow the slab layout (build_slab_tables).
+    void alloc_cands() {
+        child_scratch.alloc(static_cast<size_t>(child_rows()) * std::max<uint32_t>(ncgb, 1) * 2048);
+        child_counts.alloc(static_cast<size_t>(child_rows()) * std::max<uint32_t>(ncgb, 1));
+        hip_check(hipMemsetAsync(child_counts.p, 0, child_counts.n * sizeof(uint32_t), stream), "zero share counters");
+        const size_t n = static_cast<size_t>(JMAX) * 2 * nslot();
+        d_cands.alloc(n);
+        d_cand_gain.alloc(n);
+        d_cand_feat.alloc(n);
     }
 
     // Tile status words carry the step's epoch; the counters are returned to zero by the kernels themselves.
@@ -2044,7 +2090,10 @@ struct Context {
         g.leaf_left = d_leaf_left.p;
         g.splittable = d_splittable.p;
         g.jobs = d_jobs.p;
+        g.root_cands = d_root_cands.p;
         g.cands = d_cands.p;
+        g.cand_gain = d_cand_gain.p;
+        g.cand_feat = d_cand_feat.p;
         g.evaluate = d_eval.p;
         g.mask = d_mask.p;
         g.feats = dfeats.p;
@@ -2069,8 +2118,10 @@ struct Context {
         g.dsc = grow_dsc;
         g.target_groups = step_target;
         g.jcap = grow_jcap(spec.num_leaves);
-        g.ncg = ncg;
-        g.nsg = nsg;
+        g.ncgb = ncgb;
+        g.ncgw = ncgw;
+        g.nwide = nwide;
+        g.nslot = nslot();
         g.flush_rows = flush_rows();
         // a workgroup's i32 sums take at most (2^31 - 1) / max_q rows
         const uint64_t mq = static_cast<uint64_t>(std::max<int64_t>(std::max(max_gq, max_hq), 1));
@@ -2379,17 +2430,26 @@ void Context::grow(const srocm_grow_spec &spec, HostTree &tree, std::vector<sroc
                     prof.step_launches += static_cast<double>(launches);
                     sector_model(parity);
                 }
-                ReduceStepArgs ra{step_partial.p, d_fmt.p, d_cgs.p, d_plans.p + parity, slab_slot_flat.p};
-                k_step_reduce<<<reduce_blocks(), 256, 0, stream>>>(g, ra);
-                launch_check("k_step_reduce");
-                ScanStepArgs sca{unit_feat.p, unit_segl.p, nseg_units, cat_feats.p, ncat, d_plans.p + parity};
-                if (has_narrow64) k_step_scan<false><<<scan_blocks(), 256, 0, stream>>>(g, sca);
-                if (has_seg_units) k_step_scan_seg<<<scan_blocks(), 256, 0, stream>>>(g, sca);
-                if (has_wide) k_step_scan<true><<<scan_blocks(), 256, 0, stream>>>(g, sca);
-                launch_check("k_step_scan");
-                if (ncat) {
-                    k_step_cat<<<std::min<uint32_t>(cus * 2, div_up(static_cast<uint64_t>(JMAX) * 2 * ncat, 4)), 256, 0, stream>>>(g, sca);
-                    launch_check("k_step_cat");
+                if (ncgb) {
+                    const ChildArgs ca{step_partial.p, d_fmt.p, d_cgs.p, slab_slot_flat.p, unit_recs.p, unit_segl.p, d_plans.p + parity,
+                                       child_scratch.p, child_counts.p};
+                    const uint32_t grid = child_shares(g.jcap) * ncgb;
+                    if (has_seg_units) {
+                        if (has_cat) k_step_children<true, true><<<grid, 512, 0, stream>>>(g, ca);
+                        else k_step_children<true, false><<<grid, 512, 0, stream>>>(g, ca);
+                    } else {
+                        if (has_cat) k_step_children<false, true><<<grid, 512, 0, stream>>>(g, ca);
+                        else k_step_children<false, false><<<grid, 512, 0, stream>>>(g, ca);
+                    }
+                    launch_check("k_step_children");
+                }
+                if (nwide) {
+                    const ReduceStepArgs ra{step_partial.p, d_fmt.p, d_cgs.p + ncgb, d_plans.p + parity};
+                    k_step_reduce<<<reduce_blocks(), 256, 0, stream>>>(g, ra);
+                    launch_check("k_step_reduce");
+                    const ScanStepArgs sca{wide_feats.p, d_plans.p + parity};
+                    k_step_scan<<<scan_blocks(), 256, 0, stream>>>(g, sca);
+                    launch_check("k_step_scan");
                 }
                 SelectArgs sa2{fin_counts.p, d_plans.p + parity, d_plans.p + (parity ^ 1u)};
                 if (L <= LEAVES_SMALL) k_step_select<LEAVES_SMALL><<<g.jcap, 512, 0, stream>>>(g, sa2);

@@ -1357,6 +1357,22 @@ __device__ __forceinline__ bool candidate_stop(const Ctx &c, const SplitCfgDev &
     return other_small && !skip;
 }
 
+// Where a scan reads a feature's units from: a histogram in memory ({g, h} i64 per bin), or a child's histogram in LDS
+// (k_step_children: g and h planes of doubles, every value an exact integer).
+struct MemUnits {
+    const int64_t *p;  // the feature's bin 0
+    __device__ __forceinline__ double g(int b) const { return static_cast<double>(p[2 * b]); }
+    __device__ __forceinline__ double h(int b) const { return static_cast<double>(p[2 * b + 1]); }
+};
+struct LdsUnits {
+    const double *pg, *ph;
+    __device__ __forceinline__ double g(int b) const { return pg[b]; }
+    __device__ __forceinline__ double h(int b) const { return ph[b]; }
+};
+__device__ __forceinline__ MemUnits feature_units(const int64_t *hist, const FeatDev &m) {
+    return MemUnits{hist + 2 * static_cast<size_t>(m.hist_offset)};
+}
+
 constexpr uint32_t UNIT_FEATS = 16;  // features a scan unit holds at most (segments of 4 lanes)
 
 // A scan's lanes: the wave (SEGL = 64), or segments of SEGL = 16 or 4 lanes, each scanning its own feature of at most
@@ -1587,11 +1603,10 @@ __device__ void scan_numerical_wide(const Ctx &c, const SplitCfgDev &cfg, const 
 //   highest b on equal gains. Threshold b - 1.
 // - Forward (missing values go right; two-way features only): visits b = 0 .. top; stops at the lowest such b;
 //   keeps the lowest b on equal gains. Threshold b.
-template <int SEGL = 64>
-__device__ void scan_numerical(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const int64_t *hist, bool &rf,
-                               Grown &rg, bool &ff, Grown &fg) {
+template <int SEGL = 64, class Units>
+__device__ __forceinline__ void scan_numerical(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const Units &u, bool &rf,
+                                               Grown &rg, bool &ff, Grown &fg) {
     const int lane = static_cast<int>(threadIdx.x & static_cast<uint32_t>(SEGL - 1));  // the lane in its segment
-    const int64_t *h = hist + 2 * static_cast<size_t>(m.hist_offset);
     const int nb = static_cast<int>(m.num_bins);
     const bool two = scan_two_way(m);
     const int top = two ? nb - 2 : nb - 1;
@@ -1600,8 +1615,8 @@ __device__ void scan_numerical(const Ctx &c, const SplitCfgDev &cfg, const FeatD
     for (int j = 0; j < 4; ++j) {
         const int b = 4 * lane + j;
         const int t = b <= top ? b : 0;
-        gu[j] = b <= top ? static_cast<double>(h[2 * t]) : 0.0;
-        hu[j] = b <= top ? static_cast<double>(h[2 * t + 1]) : 0.0;
+        gu[j] = b <= top ? u.g(t) : 0.0;
+        hu[j] = b <= top ? u.h(t) : 0.0;
     }
     // per-bin counts: `(x + 0.5) as i64`, one conversion when the wave's are all in u32
     double xc[4];
@@ -1619,9 +1634,10 @@ __device__ void scan_numerical(const Ctx &c, const SplitCfgDev &cfg, const FeatD
 #pragma unroll
         for (int j = 0; j < 4; ++j) ci[j] = sat_i64(xc[j]);
     }
-    // inclusive prefix P(b) over bins 0 .. top
-    double pg[4], ph[4];
-    int64_t pc[4];
+    // inclusive prefix P(b) over bins 0 .. top, after the lane's exclusive one: p[j] is below bin 4 lane + j, p[j + 1]
+    // up to it
+    double pg[5], ph[5];
+    int64_t pc[5];
     double lg = 0.0, lh = 0.0;
     int64_t lc = 0;
 #pragma unroll
@@ -1629,107 +1645,101 @@ __device__ void scan_numerical(const Ctx &c, const SplitCfgDev &cfg, const FeatD
         lg += gu[j];
         lh += hu[j];
         lc += ci[j];
-        pg[j] = lg;
-        ph[j] = lh;
-        pc[j] = lc;
     }
     double eg = lg, eh = lh;
     int64_t ec = lc;
     seg_scan_add<SEGL>(eg, eh, ec);
     const double tg = seg_read_f64<SEGL>(eg, SEGL - 1), th = seg_read_f64<SEGL>(eh, SEGL - 1);
     const int64_t tc = seg_read_i64<SEGL>(ec, SEGL - 1);
-    eg -= lg;
-    eh -= lh;
-    ec -= lc;
-    const int64_t min_count = cfg.min_data_in_leaf > 1 ? cfg.min_data_in_leaf : 1;
-    double rgu[4], rhu[4], grv[4], gfv[4];
-    int64_t rcu[4];
-    int stop_r = -1, stop_f = 0x7fffffff;
+    pg[0] = eg - lg;
+    ph[0] = eh - lh;
+    pc[0] = ec - lc;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int b = 4 * lane + j;
-        pg[j] += eg;
-        ph[j] += eh;
-        pc[j] += ec;
-        // reverse: the right side from bin b up
-        rgu[j] = tg - (pg[j] - gu[j]);
-        rhu[j] = th - (ph[j] - hu[j]);
-        rcu[j] = tc - (pc[j] - ci[j]);
-        grv[j] = -__builtin_inf();
-        gfv[j] = -__builtin_inf();
-        if (b <= top) {
-            bool stop = false;
-            if (b >= 1) {
-                grv[j] = candidate_gain(c, cfg, rgu[j], rhu[j], rcu[j], min_count, stop);
-                if (stop) stop_r = b;  // b grows with j: the lane's highest
-            }
-            if (two) {
-                gfv[j] = candidate_gain(c, cfg, pg[j], ph[j], pc[j], min_count, stop);
-                if (stop && stop_f == 0x7fffffff) stop_f = b;  // the lane's lowest
-            }
-        }
+        pg[j + 1] = pg[j] + gu[j];
+        ph[j + 1] = ph[j] + hu[j];
+        pc[j + 1] = pc[j] + ci[j];
     }
+    const int64_t min_count = cfg.min_data_in_leaf > 1 ? cfg.min_data_in_leaf : 1;
     rf = false;
     ff = false;
-    {  // reverse: candidates above the highest stop, the highest b among equal gains
-        const int lo = seg_max_i32<SEGL>(stop_r) + 1;  // >= 0
+    {  // reverse: the right side from bin b up; candidates above the highest stop, the highest b among equal gains
+        double gain[4];
+        int stop_b = -1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int b = 4 * lane + j;
+            bool stop = false;
+            gain[j] = candidate_gain(c, cfg, tg - pg[j], th - ph[j], tc - pc[j], min_count, stop);
+            if (stop && b >= 1 && b <= top) stop_b = b;  // b grows with j: the lane's highest
+        }
+        const int lo = max(seg_max_i32<SEGL>(stop_b) + 1, 1);
         double bg = -__builtin_inf();
         int bb = -1;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int b = 4 * lane + j;
-            if (b >= 1 && b >= lo && b <= top && (bb < 0 || grv[j] >= bg)) {
-                bg = grv[j];
+            if (b >= lo && b <= top && (bb < 0 || gain[j] >= bg)) {
+                bg = gain[j];
                 bb = b;
             }
         }
-        const double best = seg_max_f64<SEGL>(bb >= 0 ? bg : -__builtin_inf());
+        const double best = seg_max_f64<SEGL>(bg);
         const int first = seg_max_i32<SEGL>(bb >= 0 && bg == best ? bb : -1);
         if (first >= 0 && best > c.min_gain_shift) {
             const uint32_t owner = static_cast<uint32_t>(first) >> 2;
             const int jj = first & 3;
-            double og = 0.0, oh = 0.0;
-            int64_t oc = 0;
+            double og = pg[0], oh = ph[0];
+            int64_t oc = pc[0];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 1; j < 4; ++j)
                 if (j == jj) {
-                    og = rgu[j];
-                    oh = rhu[j];
-                    oc = rcu[j];
+                    og = pg[j];
+                    oh = ph[j];
+                    oc = pc[j];
                 }
-            rg.ug = seg_read_f64<SEGL>(og, owner);
-            rg.uh = seg_read_f64<SEGL>(oh, owner);
-            rg.count = seg_read_i64<SEGL>(oc, owner);
+            rg.ug = tg - seg_read_f64<SEGL>(og, owner);
+            rg.uh = th - seg_read_f64<SEGL>(oh, owner);
+            rg.count = tc - seg_read_i64<SEGL>(oc, owner);
             rg.gain = best;
             rg.bin = static_cast<uint32_t>(first);
             rf = true;
         }
     }
     if (two) {  // forward: candidates below the lowest stop, the lowest b among equal gains
-        const int hi = seg_min_i32<SEGL>(stop_f);
+        double gain[4];
+        int stop_b = 0x7fffffff;
+#pragma unroll
+        for (int j = 3; j >= 0; --j) {
+            const int b = 4 * lane + j;
+            bool stop = false;
+            gain[j] = candidate_gain(c, cfg, pg[j + 1], ph[j + 1], pc[j + 1], min_count, stop);
+            if (stop && b <= top) stop_b = b;  // b falls with j: the lane's lowest
+        }
+        const int hi = seg_min_i32<SEGL>(stop_b);
         double bg = -__builtin_inf();
         int bb = -1;
 #pragma unroll
         for (int j = 3; j >= 0; --j) {
             const int b = 4 * lane + j;
-            if (b < hi && b <= top && (bb < 0 || gfv[j] >= bg)) {
-                bg = gfv[j];
+            if (b < hi && b <= top && (bb < 0 || gain[j] >= bg)) {
+                bg = gain[j];
                 bb = b;
             }
         }
-        const double best = seg_max_f64<SEGL>(bb >= 0 ? bg : -__builtin_inf());
+        const double best = seg_max_f64<SEGL>(bg);
         const int first = seg_min_i32<SEGL>(bb >= 0 && bg == best ? bb : 0x7fffffff);
         if (first != 0x7fffffff && best > c.min_gain_shift) {
             const uint32_t owner = static_cast<uint32_t>(first) >> 2;
             const int jj = first & 3;
-            double og = 0.0, oh = 0.0;
-            int64_t oc = 0;
+            double og = pg[1], oh = ph[1];
+            int64_t oc = pc[1];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 1; j < 4; ++j)
                 if (j == jj) {
-                    og = pg[j];
-                    oh = ph[j];
-                    oc = pc[j];
+                    og = pg[j + 1];
+                    oh = ph[j + 1];
+                    oc = pc[j + 1];
                 }
             fg.ug = seg_read_f64<SEGL>(og, owner);
             fg.uh = seg_read_f64<SEGL>(oh, owner);
@@ -1807,8 +1817,8 @@ __device__ __forceinline__ void mask_set(uint32_t (&mask)[8], uint32_t bin) {
 
 // split.rs:695-736 find_onehot: every bin 1..num_bins on its own against the rest; the first strict maximum above
 // min_gain_shift (NaN never counts). Lane l takes bins 1 + l + 64 j.
-__device__ FeatCand onehot_scan(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const int64_t *hist) {
-    const int64_t *h = hist + 2 * static_cast<size_t>(m.hist_offset);
+template <class Units>
+__device__ FeatCand onehot_scan(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const Units &u) {
     const uint32_t lane = threadIdx.x & 63u;
     const int nb = static_cast<int>(m.num_bins);
     double bg = 0.0, bu_g = 0.0, bu_h = 0.0;
@@ -1818,7 +1828,7 @@ __device__ FeatCand onehot_scan(const Ctx &c, const SplitCfgDev &cfg, const Feat
     for (int j = 0; j < 4; ++j) {
         const int t = 1 + static_cast<int>(lane) + 64 * j;
         if (t >= nb) continue;
-        const double ug = static_cast<double>(h[2 * t]), uh = static_cast<double>(h[2 * t + 1]);
+        const double ug = u.g(t), uh = u.h(t);
         const int64_t cnt = bin_rows(c, uh);
         const double raw_hess = uh * c.scale_hess;
         const int64_t other_cnt = c.num_data - cnt;
@@ -1882,7 +1892,8 @@ __device__ __forceinline__ unsigned long long total_order_bits(double x) {
 // One run of split.rs:795-843 SortedScan::run over the first `steps` positions of the sorted order, from the low
 // end (forward) or the high end. Positions i = lane + 64 j; the stateful min_data_per_group walk is uniform.
 // Returns whether a candidate passed; (gain, pos) the best, and its left sums.
-__device__ bool sorted_run(const Ctx &c, const SplitCfgDev &cfg, const int64_t *h, const CatScratch &sc, int used,
+template <class Units>
+__device__ bool sorted_run(const Ctx &c, const SplitCfgDev &cfg, const Units &u, const CatScratch &sc, int used,
                            int steps, bool forward, double l2, bool &splittable, double &best_gain, int &best_pos,
                            double &lug, double &luh, int64_t &lcnt) {
     const uint32_t lane = threadIdx.x & 63u;
@@ -1897,8 +1908,8 @@ __device__ bool sorted_run(const Ctx &c, const SplitCfgDev &cfg, const int64_t *
         int64_t cn = 0;
         if (i < steps) {
             const uint32_t t = sc.order[forward ? i : used - 1 - i];
-            gu = static_cast<double>(h[2 * t]);
-            hu = static_cast<double>(h[2 * t + 1]);
+            gu = u.g(static_cast<int>(t));
+            hu = u.h(static_cast<int>(t));
             cn = bin_rows(c, hu);
         }
         ci[j] = cn;
@@ -1985,9 +1996,9 @@ __device__ bool sorted_run(const Ctx &c, const SplitCfgDev &cfg, const int64_t *
 }
 
 // split.rs:740-784: sorted categorical. `order_out` (when given) receives the left bins in the rule's order.
-__device__ FeatCand sorted_scan(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const int64_t *hist,
-                                CatScratch &sc, uint8_t *order_out) {
-    const int64_t *h = hist + 2 * static_cast<size_t>(m.hist_offset);
+template <class Units>
+__device__ FeatCand sorted_scan(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const Units &u, CatScratch &sc,
+                                uint8_t *order_out) {
     const uint32_t lane = threadIdx.x & 63u;
     const int nb = static_cast<int>(m.num_bins < 256 ? m.num_bins : 256);
     // split.rs:740-760: bins with at least cat_smooth (estimated) rows, by (g / (h + cat_smooth), bin)
@@ -1999,7 +2010,7 @@ __device__ FeatCand sorted_scan(const Ctx &c, const SplitCfgDev &cfg, const Feat
         ok[j] = false;
         key[j] = 0;
         if (t < nb) {
-            const double gu = static_cast<double>(h[2 * t]), hu = static_cast<double>(h[2 * t + 1]);
+            const double gu = u.g(t), hu = u.h(t);
             ok[j] = static_cast<double>(bin_rows(c, hu)) >= cfg.cat_smooth;
             key[j] = total_order_bits((gu * c.scale_grad) / (hu * c.scale_hess + cfg.cat_smooth));
         }
@@ -2020,9 +2031,9 @@ __device__ FeatCand sorted_scan(const Ctx &c, const SplitCfgDev &cfg, const Feat
         const int t = 1 + static_cast<int>(lane) + 64 * j;
         int rank = 0;
         if (ok[j])
-            for (int u = 1; u < nb; ++u) {
-                const unsigned long long ku = sc.key[u];
-                rank += (sc.eligible[u] && (ku < key[j] || (ku == key[j] && u < t))) ? 1 : 0;
+            for (int v = 1; v < nb; ++v) {
+                const unsigned long long kv = sc.key[v];
+                rank += (sc.eligible[v] && (kv < key[j] || (kv == key[j] && v < t))) ? 1 : 0;
             }
         __builtin_amdgcn_wave_barrier();
         if (ok[j]) sc.order[rank] = static_cast<uint32_t>(t);
@@ -2038,8 +2049,8 @@ __device__ FeatCand sorted_scan(const Ctx &c, const SplitCfgDev &cfg, const Feat
     double fg = 0.0, bgn = 0.0, flg = 0.0, flh = 0.0, blg = 0.0, blh = 0.0;
     int fp = -1, bpz = -1;
     int64_t flc = 0, blc = 0;
-    const bool ff = steps > 0 && sorted_run(c, cfg, h, sc, used, steps, true, l2, splittable, fg, fp, flg, flh, flc);
-    const bool bf = steps > 0 && sorted_run(c, cfg, h, sc, used, steps, false, l2, splittable, bgn, bpz, blg, blh, blc);
+    const bool ff = steps > 0 && sorted_run(c, cfg, u, sc, used, steps, true, l2, splittable, fg, fp, flg, flh, flc);
+    const bool bf = steps > 0 && sorted_run(c, cfg, u, sc, used, steps, false, l2, splittable, bgn, bpz, blg, blh, blc);
     r.splittable = splittable ? 1 : 0;
     if (!ff && !bf) return r;
     const bool fwd = ff && !(bf && bgn > fg);  // split.rs:775-781: the backward run replaces only a lower gain
@@ -2069,10 +2080,11 @@ __device__ FeatCand sorted_scan(const Ctx &c, const SplitCfgDev &cfg, const Feat
 }
 
 // The candidate of a categorical feature (split.rs:847-862).
+template <class Units>
 __device__ __forceinline__ FeatCand categorical_candidate(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m,
-                                                          const int64_t *hist, CatScratch &sc, uint8_t *order_out) {
-    if (m.num_bins <= cfg.max_cat_to_onehot) return onehot_scan(c, cfg, m, hist);
-    return sorted_scan(c, cfg, m, hist, sc, order_out);
+                                                          const Units &u, CatScratch &sc, uint8_t *order_out) {
+    if (m.num_bins <= cfg.max_cat_to_onehot) return onehot_scan(c, cfg, m, u);
+    return sorted_scan(c, cfg, m, u, sc, order_out);
 }
 
 // split.rs:584-620 find_numerical (or a categorical search) for one feature of one leaf, by one wave. WIDE: the
@@ -2087,8 +2099,9 @@ __device__ FeatCand scan_feature(const Ctx &c, const SplitCfgDev &cfg, const Fea
     if constexpr (WIDE) {
         scan_numerical_wide(c, cfg, m, hist, rf, rg, ff, fg);
     } else {
-        if (m.kind == 2) return categorical_candidate(c, cfg, m, hist, sc, order_out);
-        scan_numerical(c, cfg, m, hist, rf, rg, ff, fg);
+        const MemUnits u = feature_units(hist, m);
+        if (m.kind == 2) return categorical_candidate(c, cfg, m, u, sc, order_out);
+        scan_numerical(c, cfg, m, u, rf, rg, ff, fg);
     }
     return feature_candidate(c, m, rf, rg, ff, fg);
 }
@@ -2116,24 +2129,25 @@ __global__ __launch_bounds__(256) void k_split_scan(const ScanJob *__restrict__ 
     if ((threadIdx.x & 63) == 0) job.out[f] = r;
 }
 
-// k_split_scan for scan units of several numerical byte features of at most 64 bins (16 or 4 lanes a feature, as
-// k_step_scan_seg): unit u holds unit_feat[u * UNIT_FEATS ...] (-1 padding), unit_segl[u] lanes each. A wave per
+// k_split_scan for scan units of several numerical byte features of at most 64 bins (16 or 4 lanes a feature, as in
+// k_step_children): unit u holds unit_feat[u * UNIT_FEATS ...] (-1 padding), unit_segl[u] lanes each. A wave per
 // unit and job. grid: (ceil(units / 4), jobs), 256 threads.
 __global__ __launch_bounds__(256) void k_split_scan_seg(const ScanJob *__restrict__ jobs, const FeatDev *__restrict__ feats,
                                                         const uint8_t *__restrict__ evaluate, const int32_t *unit_feat,
-                                                        const uint32_t *unit_segl, uint32_t units, SplitCfgDev cfg,
+                                                        const uint32_t *unit_segl, uint32_t num_units, SplitCfgDev cfg,
                                                         double sg, double sh) {
     const ScanJob &job = jobs[blockIdx.y];
     const uint32_t u = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
-    if (u >= units) return;
+    if (u >= num_units) return;
     const uint32_t segl = unit_segl[u];  // 16 or 4, wave-uniform
     const int32_t f = unit_feat[u * UNIT_FEATS + lane / segl];
     const FeatDev m = f >= 0 ? feats[f] : FeatDev{};
     const Ctx c = make_ctx(cfg, sg, sh, job.units_grad, job.units_hess, job.count);
     Grown rg = {}, fg = {};
     bool rf = false, ff = false;
-    if (segl == 16u) scan_numerical<16>(c, cfg, m, job.hist, rf, rg, ff, fg);
-    else scan_numerical<4>(c, cfg, m, job.hist, rf, rg, ff, fg);
+    const MemUnits units = feature_units(job.hist, m);
+    if (segl == 16u) scan_numerical<16>(c, cfg, m, units, rf, rg, ff, fg);
+    else scan_numerical<4>(c, cfg, m, units, rf, rg, ff, fg);
     FeatCand r = {};
     if (f >= 0 && scan_searched(c, m, evaluate[f] != 0)) r = feature_candidate(c, m, rf, rg, ff, fg);
     if ((lane & (segl - 1u)) == 0 && f >= 0) job.out[f] = r;
@@ -2376,8 +2390,8 @@ struct JobPlan {
     uint32_t groups, group_base;  // k_step_rows workgroups, one partial each
     uint32_t packed;              // the partials are packed 16/16 LDS words (one tile per workgroup)
     uint32_t ways;                // k_step_reduce stripes of the partials (reduce_ways)
-    uint32_t red_base, red_items; // k_step_reduce work items: per column group, `ways` (packed) or 4 * `ways`
-    uint32_t scan_base, scan_items;  // k_step_scan work items: a scan per column group (when histogrammed)
+    uint32_t red_base;            // k_step_reduce work items: per column group of two-byte slabs, `ways`
+    uint32_t scan_base;           // k_step_scan work items: one per two-byte feature
     uint32_t ticket;              // next partition tile to hand out
     uint32_t left;                // rows going left, written by the last tile
     int32_t kid;                  // the children's speculative leaves
@@ -2385,16 +2399,35 @@ struct JobPlan {
     double child_ug[2], child_uh[2];  // the children's sums in histogram units (left, right)
 };
 
+// What k_step_children needs of a histogrammed job, found by its item's index alone (item / column groups), so that a
+// block's first loads do not wait for a search of the jobs. A job of more than CHILD_SPLIT partials has a record for each
+// of `ways` shares of about CHILD_SHARE partials, whose sums meet in scratch: in a tree's first step one job has a partial
+// a compute unit, and one block a column group left most of the chip idle (88 us a launch on
+// 10M x 128, 39 with shares; at 100 partials a job, the meeting cost more than it saved: 24 us against 34).
+constexpr uint32_t CHILD_SPLIT = 160, CHILD_SHARE = 32, CHILD_WAYS = 16;  // a job's shares at most
+constexpr uint32_t CHILD_MAX = JMAX + 64;                                // records of a step at most
+struct ChildJob {
+    uint32_t j, t, built_side;      // the job, its leaf, the histogrammed child
+    uint32_t group_base, groups;    // the share's partials
+    uint32_t ways, way, scratch;    // the job's shares, this one, the first one's scratch and counter row
+    int32_t parent_slot, built_slot, kid;
+    int64_t parent_count;
+    double child_ug[2], child_uh[2];
+};
+
 // A split step: the plan of step s is plans[s % 2], written by the step before it.
 struct StepPlan {
     uint32_t njobs;
     uint32_t total_groups;  // k_step_rows workgroups in use
+    uint32_t total_child;   // k_step_children work items
     uint32_t total_red;     // k_step_reduce work items
     uint32_t total_scan;    // k_step_scan work items
     uint32_t epoch;         // tags the step's tile status words
-    uint32_t pad_[3];
-    // the jobs' first workgroup, reduce item and scan item side by side (a job search reads one run of words)
+    uint32_t pad_[2];
+    // the jobs' first workgroup and work items side by side (a job search reads one run of words)
     uint32_t group_base[JMAX], red_base[JMAX], scan_base[JMAX];
+    uint32_t pairs[JMAX];   // some partial of the job is {g, h} pairs (set by k_step_rows)
+    ChildJob child[CHILD_MAX];  // the histogrammed jobs' shares
     JobPlan jobs[JMAX];
 };
 
@@ -2442,7 +2475,11 @@ struct GrowState {
     uint8_t *leaf_left;       // [num_leaves]: the committed leaf is its parent's left child
     uint8_t *splittable;      // [tcap][nf]
     ScanJob *jobs;            // [1]: the root's search
-    FeatCand *cands;          // [JMAX][2][nf]
+    FeatCand *root_cands;     // [nf]: the root's search
+    FeatCand *cands;          // [JMAX][2][nslot]: a step's children's candidates, the best of each column group of byte
+                              // slabs, then each two-byte feature's
+    double *cand_gain;        // their gains (NaN as -inf) and features (-1: none), apart for coalesced loads
+    int32_t *cand_feat;
     uint8_t *evaluate;        // [nf]: the root's evaluated features
     const uint8_t *mask;      // [nf], the tree's feature mask
     const FeatDev *feats;
@@ -2457,8 +2494,10 @@ struct GrowState {
     const struct DevScales *dsc;  // when set, the scales are these (made on the device), not sg and sh
     uint32_t target_groups;   // k_step_rows workgroups a step is spread over
     uint32_t jcap;            // jobs a step at most: grow_jcap(num_leaves)
-    uint32_t ncg;             // column groups of k_step_reduce
-    uint32_t nsg;             // scan units of k_step_scan (a wave per unit and child)
+    uint32_t ncgb;            // column groups of byte slabs (k_step_children), the first ones
+    uint32_t ncgw;            // column groups of two-byte slabs (k_step_reduce)
+    uint32_t nwide;           // two-byte features (k_step_scan, a wave per feature and child)
+    uint32_t nslot;           // ncgb + nwide
     uint32_t flush_rows;      // rows a packed 16/16 LDS word can take
     uint32_t tile_cap;        // k_step_rows tiles a workgroup may take (its i32 sums of the quantized units)
     float hist_weight;        // the planner's cost of a tile of histogrammed rows, in partitioned tiles of a dense
@@ -2578,6 +2617,7 @@ __global__ void k_grow_init(GrowState g, uint32_t root_begin, uint32_t root_coun
         for (int k = 0; k < 2; ++k) {
             g.plans[k].njobs = 0;
             g.plans[k].total_groups = 0;
+            g.plans[k].total_child = 0;
             g.plans[k].total_red = 0;
             g.plans[k].total_scan = 0;
         }
@@ -2618,7 +2658,7 @@ __global__ __launch_bounds__(256) void k_root_prep(GrowState g) {
         const double dg = static_cast<double>(tg), dh = static_cast<double>(th);
         g.tl[0].ug = dg;
         g.tl[0].uh = dh;
-        g.jobs[0] = ScanJob{h, dg, dh, l.cnt, g.cands};
+        g.jobs[0] = ScanJob{h, dg, dh, l.cnt, g.root_cands};
     }
 }
 
@@ -3639,24 +3679,25 @@ __device__ void advance(const GrowState &g, StepPlan &next, void *scratch) {
         }
         const uint32_t groups_before = wave_excl_sum(groups);
         const uint32_t total_groups = wave_total(groups);
-        uint32_t red = 0, scan = 0;
+        uint32_t red = 0;
         if (on) {
             J.tile_base = tiles_before;
             J.groups = groups;
             J.group_base = groups_before;
             J.packed = (ntiles <= groups && g.flush_rows >= STEP_TILE) ? 1u : 0u;
             J.ways = reduce_ways(groups);
-            red = hist ? g.ncg * J.ways : 0u;
-            scan = hist ? g.nsg : 0u;
-            J.red_items = red;
-            J.scan_items = scan;
+            red = hist ? g.ncgw * J.ways : 0u;
             J.built_slot = hist ? static_cast<int32_t>(slot0 + hist_before) : -1;
         }
-        const uint32_t red_before = wave_excl_sum(red), scan_before = wave_excl_sum(scan);
-        const uint32_t total_red = wave_total(red), total_scan = wave_total(scan);
+        const uint32_t red_before = wave_excl_sum(red), total_red = wave_total(red);
         const uint32_t nhist = wave_total(hist);
+        uint32_t ways = hist ? (groups > CHILD_SPLIT ? min(CHILD_WAYS, (groups + CHILD_SHARE - 1) / CHILD_SHARE) : 1u) : 0u;
+        if (wave_total(ways) > CHILD_MAX) ways = hist;  // uniform
+        const uint32_t share_before = wave_excl_sum(ways), total_shares = wave_total(ways);
+        const uint32_t scratch_before = wave_excl_sum(ways > 1u ? ways : 0u);
         if (on) {
             J.red_base = red_before;
+            const uint32_t scan_before = hist_before * g.nwide;
             J.scan_base = scan_before;
             next.group_base[lane] = J.group_base;
             next.red_base[lane] = red_before;
@@ -3664,6 +3705,14 @@ __device__ void advance(const GrowState &g, StepPlan &next, void *scratch) {
             J.ticket = 0;
             J.left = 0;
             next.jobs[lane] = J;
+            next.pairs[lane] = 0;
+            const uint32_t per = ways ? (groups + ways - 1) / ways : 0u;
+            for (uint32_t w = 0; w < ways; ++w) {
+                const uint32_t b = min(w * per, groups);
+                next.child[share_before + w] = ChildJob{lane, J.t, J.built_side, J.group_base + b, min(per, groups - b), ways, w, scratch_before,
+                                                        J.parent_slot, J.built_slot, J.kid, J.parent_count,
+                                                        {J.child_ug[0], J.child_ug[1]}, {J.child_uh[0], J.child_uh[1]}};
+            }
             g.tl[J.t].state = T_PLANNED;
             g.tl[J.t].kid = J.kid;
             g.tk[J.t].state = T_PLANNED;
@@ -3672,8 +3721,9 @@ __device__ void advance(const GrowState &g, StepPlan &next, void *scratch) {
         if (lane == 0) {
             next.njobs = njobs;
             next.total_groups = total_groups;
+            next.total_child = total_shares * g.ncgb;
             next.total_red = total_red;
-            next.total_scan = total_scan;
+            next.total_scan = nhist * g.nwide;
             next.epoch = epoch0 + 1;
             ctl->epoch = epoch0 + 1;
             ctl->ntent = ntent + 2 * njobs;
@@ -3755,9 +3805,9 @@ __global__ __launch_bounds__(512) void k_root_select(GrowState g) {
 // both children are stable; a leaf stored last-first is read back to front by the step that expands it and by
 // k_consolidate. Launches for a second or later slab only histogram.
 //
-// Then, one launch each: k_step_reduce adds each job's partials (work items: job, column group, bin range), writes
-// the built child's histogram and forms the sibling by subtraction (learner.rs:356-371); k_step_scan and
-// k_step_cat scan every (job, feature, child); k_step_select selects both children's splits of each job
+// Then, one launch each: k_step_children adds each job's partials, writes the built child's histogram, forms the sibling
+// by subtraction (learner.rs:356-371) and scans every (job, feature, child) of the byte slabs (k_step_reduce and
+// k_step_scan do so for two-byte slabs); k_step_select selects both children's splits of each job
 // (job_select), and its last block to finish runs advance. That hand-off is a counter the last arriving block
 // resets; no block ever waits for another.
 // ---------------------------------------------------------------------------------------------------------
@@ -3830,36 +3880,82 @@ __device__ uint32_t lookback(const unsigned long long *status, uint32_t t, uint3
     return prefix;
 }
 
-// Moves the packed 16/16 LDS words (Q32: the separate g and h counters) into a workgroup's {g, h} pair partial
-// (stored, or added to what an earlier flush stored) and zeroes them. Slot tid + 1024 j is bin (tid + 1024 j) / W
-// of column tid % W; bins past the column's feature are not stored. Block-wide.
+// The 4 x 4 transpose of a quad of lanes' v[0 .. 3]: lane c4 = lane % 4 leaves with v[c4] of lanes 0 .. 3 of its quad. At
+// level b a lane keeps the elements whose index bit b matches its own and swaps the other two with lane c4 ^ b; every
+// choice is one select on a lane bit.
+__device__ __forceinline__ int4 quad_transpose(int32_t v0, int32_t v1, int32_t v2, int32_t v3) {
+    const uint32_t c4 = threadIdx.x & 3u;
+    {
+        const bool hi = (c4 & 1u) != 0;
+        const int32_t t0 = __builtin_amdgcn_update_dpp(0, hi ? v0 : v1, 0xB1, 0xf, 0xf, false);
+        const int32_t t1 = __builtin_amdgcn_update_dpp(0, hi ? v2 : v3, 0xB1, 0xf, 0xf, false);
+        const int32_t n0 = hi ? t0 : v0, n1 = hi ? v1 : t0, n2 = hi ? t1 : v2, n3 = hi ? v3 : t1;
+        v0 = n0;
+        v1 = n1;
+        v2 = n2;
+        v3 = n3;
+    }
+    {
+        const bool hi = (c4 & 2u) != 0;
+        const int32_t t0 = __builtin_amdgcn_update_dpp(0, hi ? v0 : v2, 0x4E, 0xf, 0xf, false);
+        const int32_t t1 = __builtin_amdgcn_update_dpp(0, hi ? v1 : v3, 0x4E, 0xf, 0xf, false);
+        const int32_t n0 = hi ? t0 : v0, n1 = hi ? t1 : v1, n2 = hi ? v2 : t0, n3 = hi ? v3 : t1;
+        v0 = n0;
+        v1 = n1;
+        v2 = n2;
+        v3 = n3;
+    }
+    return make_int4(v0, v1, v2, v3);
+}
+
+// Moves the packed 16/16 LDS words (Q32: the separate g and h counters) into a workgroup's {g, h} partial (stored, or
+// added to what an earlier flush stored) and zeroes them. The partial is two planes, the g sums then (64 W int4s on) the
+// h sums, each in the order of a packed partial (store_packed_partial), so that a reduce's wave reads either in whole
+// lines (as {g, h} pairs bin-major, each thread's 32 bytes lay in a line of its own: the first step of a 10M x 128 tree,
+// one job over 288 such partials, took k_step_children 165 us, 88 in planes). `col_bins`: the most bins of the thread's quad
+// of columns; bins past them are not stored. Block-wide.
 template <int W, bool Q32 = false>
-__device__ __forceinline__ void flush_pairs(int32_t *lds, int2 *pairs, uint32_t col_bins, bool add) {
+__device__ __forceinline__ void flush_pairs(int32_t *lds, int4 *planes, uint32_t col_bins, bool add) {
     constexpr int SLOTS = 256 * W / 1024;
     const uint32_t tid = threadIdx.x;
     __syncthreads();
-#pragma unroll 8
-    for (int j = 0; j < SLOTS; ++j) {
-        const uint32_t slot = tid + j * 1024;
-        const int32_t v = lds[slot];
-        lds[slot] = 0;
-        int32_t gq, hq;
-        if constexpr (Q32) {
-            gq = v;
-            hq = lds[256 * W + slot];
-            lds[256 * W + slot] = 0;
-        } else {
-            gq = packed_g(v);
-            hq = packed_h(v, gq);
+#pragma unroll 2
+    for (int it = 0; it < SLOTS / 4; ++it) {
+        const uint32_t k = tid + 1024u * it, c = k % W, q = k / W;
+        int32_t gq[4], hq[4];
+#pragma unroll
+        for (uint32_t b = 0; b < 4; ++b) {
+            const uint32_t slot = (4 * q + b) * W + c;
+            const int32_t v = lds[slot];
+            lds[slot] = 0;
+            if constexpr (Q32) {
+                gq[b] = v;
+                hq[b] = lds[256 * W + slot];
+                lds[256 * W + slot] = 0;
+            } else {
+                gq[b] = packed_g(v);
+                hq[b] = packed_h(v, gq[b]);
+            }
         }
-        if (slot / W < col_bins) {
-            int2 o = add ? pairs[slot] : make_int2(0, 0);
-            o.x += gq;
-            o.y += hq;
-            pairs[slot] = o;
+        int4 g4 = quad_transpose(gq[0], gq[1], gq[2], gq[3]), h4 = quad_transpose(hq[0], hq[1], hq[2], hq[3]);
+        if (4 * q + (tid & 3u) < col_bins) {
+            int4 *pg = planes + q * W + c, *ph = pg + 64 * W;
+            if (add) {
+                const int4 og = *pg, oh = *ph;
+                g4 = make_int4(g4.x + og.x, g4.y + og.y, g4.z + og.z, g4.w + og.w);
+                h4 = make_int4(h4.x + oh.x, h4.y + oh.y, h4.z + oh.z, h4.w + oh.w);
+            }
+            *pg = g4;
+            *ph = h4;
         }
     }
     __syncthreads();
+}
+// The most bins of the thread's quad of columns (tid % W and its three neighbours), for flush_pairs.
+template <int W>
+__device__ __forceinline__ uint32_t quad_bins(const uint32_t *col_bins) {
+    const uint4 b = *reinterpret_cast<const uint4 *>(col_bins + (threadIdx.x % W & ~3u));
+    return max(max(b.x, b.y), max(b.z, b.w));
 }
 
 // A job of the step as one workgroup of k_step_rows sees it.
@@ -4067,35 +4163,12 @@ template <int W>
 __device__ __forceinline__ void store_packed_partial(const int32_t *lds, int32_t *partial) {
     constexpr int SLOTS = 256 * W / 1024;
     int4 *out = reinterpret_cast<int4 *>(partial);
-    const uint32_t tid = threadIdx.x, c4 = tid & 3u;
+    const uint32_t tid = threadIdx.x;
 #pragma unroll
     for (int it = 0; it < SLOTS / 4; ++it) {
         const uint32_t k = tid + 1024u * it, c = k % W, q = k / W;
-        int32_t v0 = lds[(4 * q + 0) * W + c], v1 = lds[(4 * q + 1) * W + c];
-        int32_t v2 = lds[(4 * q + 2) * W + c], v3 = lds[(4 * q + 3) * W + c];
-        // at level b a lane keeps the elements whose index bit b matches its own and swaps the other two with
-        // lane c4 ^ b; every choice is one select on a lane bit
-        {
-            const bool hi = (c4 & 1u) != 0;
-            const int32_t t0 = __builtin_amdgcn_update_dpp(0, hi ? v0 : v1, 0xB1, 0xf, 0xf, false);
-            const int32_t t1 = __builtin_amdgcn_update_dpp(0, hi ? v2 : v3, 0xB1, 0xf, 0xf, false);
-            const int32_t n0 = hi ? t0 : v0, n1 = hi ? v1 : t0, n2 = hi ? t1 : v2, n3 = hi ? v3 : t1;
-            v0 = n0;
-            v1 = n1;
-            v2 = n2;
-            v3 = n3;
-        }
-        {
-            const bool hi = (c4 & 2u) != 0;
-            const int32_t t0 = __builtin_amdgcn_update_dpp(0, hi ? v0 : v2, 0x4E, 0xf, 0xf, false);
-            const int32_t t1 = __builtin_amdgcn_update_dpp(0, hi ? v1 : v3, 0x4E, 0xf, 0xf, false);
-            const int32_t n0 = hi ? t0 : v0, n1 = hi ? t1 : v1, n2 = hi ? v2 : t0, n3 = hi ? v3 : t1;
-            v0 = n0;
-            v1 = n1;
-            v2 = n2;
-            v3 = n3;
-        }
-        out[q * W + c] = make_int4(v0, v1, v2, v3);  // column (c & ~3) + j at bin 4q + c4
+        // column (c & ~3) + j at bin 4q + c % 4
+        out[q * W + c] = quad_transpose(lds[(4 * q + 0) * W + c], lds[(4 * q + 1) * W + c], lds[(4 * q + 2) * W + c], lds[(4 * q + 3) * W + c]);
     }
 }
 
@@ -4250,8 +4323,8 @@ __device__ __forceinline__ void step_rows_body(const StepArgs &a, int32_t *lds, 
         const uint32_t c0 = min(nb, gi * per), c1 = min(nb, c0 + per);
         const uint32_t *list = v.dst + b0;
         const uint8_t *codes = CODES ? v.cdst + b0 : nullptr;
-        int2 *pairs = reinterpret_cast<int2 *>(R.partial) + static_cast<size_t>(wg) * step_partial_stride(W);
-        const uint32_t col_bins = (PACK > 1 || DP > 0) ? 256u : R.col_bins[tid % W];
+        int4 *pairs = reinterpret_cast<int4 *>(R.partial + 2 * static_cast<size_t>(wg) * step_partial_stride(W));
+        const uint32_t col_bins = (PACK > 1 || DP > 0) ? 256u : quad_bins<W>(R.col_bins);
         __syncthreads();  // the LDS histogram is zeroed
         bool flushed = false;
         for (uint32_t ca = c0; ca < c1;) {
@@ -4271,7 +4344,10 @@ __device__ __forceinline__ void step_rows_body(const StepArgs &a, int32_t *lds, 
             return;
         }
         flush_pairs<W, Q32>(lds, pairs, col_bins, flushed);
-        if (tid == 0) R.fmt[wg] = 0u;
+        if (tid == 0) {
+            R.fmt[wg] = 0u;
+            P.pairs[j] = 1u;
+        }
         return;
     }
 
@@ -4297,9 +4373,12 @@ __device__ __forceinline__ void step_rows_body(const StepArgs &a, int32_t *lds, 
         if (v.partition) tile_scatter<CODES>(v, t, st, sh);
         if (!v.hist) return;
         if constexpr (Q32) {  // the counters as a {g, h} pair partial
-            int2 *pairs = reinterpret_cast<int2 *>(R.partial) + static_cast<size_t>(wg) * step_partial_stride(W);
+            int4 *pairs = reinterpret_cast<int4 *>(R.partial + 2 * static_cast<size_t>(wg) * step_partial_stride(W));
             flush_pairs<W, true>(lds, pairs, 256u, false);
-            if (tid == 0) R.fmt[wg] = 0u;
+            if (tid == 0) {
+            R.fmt[wg] = 0u;
+            P.pairs[j] = 1u;
+        }
             return;
         }
         store_packed_partial<W>(lds, R.partial + 2 * static_cast<size_t>(wg) * step_partial_stride(W));
@@ -4309,9 +4388,9 @@ __device__ __forceinline__ void step_rows_body(const StepArgs &a, int32_t *lds, 
 
     // several tiles per workgroup: whenever flush_rows rows have gone into the packed words they are added into the
     // partial as {g, h} pairs; a workgroup that never flushes stores its partial packed instead
-    int2 *pairs = reinterpret_cast<int2 *>(R.partial) + static_cast<size_t>(wg) * step_partial_stride(W);
+    int4 *pairs = reinterpret_cast<int4 *>(R.partial + 2 * static_cast<size_t>(wg) * step_partial_stride(W));
     // slot tid + 1024 j is bin (tid + 1024 j) / W of column tid % W; a packed column's features are all stored
-    const uint32_t col_bins = (PACK > 1 || DP > 0) ? 256u : R.col_bins[tid % W];
+    const uint32_t col_bins = (PACK > 1 || DP > 0) ? 256u : quad_bins<W>(R.col_bins);
     uint32_t pending = 0;  // rows added to the packed LDS words since they were last flushed
     bool flushed = false;
     // partition launches take tiles in ticket order, the next ticket drawn while the current tile is worked on (a
@@ -4390,7 +4469,10 @@ __device__ __forceinline__ void step_rows_body(const StepArgs &a, int32_t *lds, 
         return;
     }
     flush_pairs<W, Q32>(lds, pairs, col_bins, flushed);
-    if (tid == 0) R.fmt[wg] = 0u;
+    if (tid == 0) {
+            R.fmt[wg] = 0u;
+            P.pairs[j] = 1u;
+        }
 }
 
 // CODES: the built rows' gradients come from the codes beside their ids (a.codes0 / a.codes1), else gathered. The
@@ -4483,7 +4565,7 @@ __global__ __launch_bounds__(256) void k_sector_bits(uint32_t *bits, uint64_t wo
     if ((threadIdx.x & 63u) == 0 && c) atomicAdd(counters + 4, c);
 }
 
-// Four columns of one slab: a work unit of k_step_reduce and k_step_scan.
+// Four columns of one slab: a work unit of k_step_children (byte slabs) or k_step_reduce (two-byte slabs).
 struct ColGroup {
     uint64_t partial;  // the slab's partials, in {g, h} pairs from the start of the step partial buffer
     uint32_t width;    // the slab's W
@@ -4495,6 +4577,8 @@ struct ColGroup {
     uint32_t seg_shift;     // a column holds a feature each 2^seg_shift bins (8: one; 7 or 6 in a packed slab)
     uint32_t dense;         // a dense slab: the slots' flat bins come from the slot table at slot_base
     uint32_t slot_base;
+    uint32_t pairs;         // the slab's partials are always {g, h} pairs (separate 32-bit counters)
+    uint32_t unit_first, unit_count;  // the columns' scan units (k_step_children); CG_COLS a group unless segmented
 };
 
 // Block-wide hand-off through `counter`: true in every thread of the block that arrives last of `target` blocks,
@@ -4519,14 +4603,30 @@ __device__ __forceinline__ bool arrive_last(uint32_t *counter, uint32_t target) 
     return s_last != 0;
 }
 
-// A scan unit is one wave's scan of a child: one feature (SEGL 64), or 4 features of at most 64 bins (SEGL 16) or
-// 16 of at most 16 bins (SEGL 4), a segment of lanes each (UNIT_FEATS entries a unit).
+// One feature of a scan unit (k_step_children): a unit is one wave's scan of a child's histogram, of one feature (64
+// lanes), or of 4 features of at most 64 bins (16 lanes each) or 16 of at most 16 bins (4 lanes each), a segment of lanes
+// each (UNIT_FEATS records a unit). `at`: the feature's bin 0 in a child's LDS planes, 256 * (column in its group) + the
+// column's row.
+struct UnitRec {
+    int32_t feat;  // -1: padding
+    uint32_t at;
+    FeatDev m;
+};
+
+struct ChildArgs {
+    const int32_t *partial;     // the step partial buffer
+    const uint32_t *fmt;        // the partials' formats (per slab, per k_step_rows workgroup: 1 packed, 0 pairs)
+    const ColGroup *cgs;        // [ncgb]
+    const uint32_t *slot_flat;  // dense slabs: per slot, its flat-histogram bin + 1 (0: none)
+    const UnitRec *recs;        // [units][UNIT_FEATS]; when no unit holds several features, [ncgb][CG_COLS]
+    const uint32_t *unit_segl;  // per unit, its lanes a feature: 64, 16 or 4
+    StepPlan *plan;
+    int64_t *scratch;           // the shares' sums: [scratch row][column group][4][512]
+    uint32_t *counters;         // [scratch row][column group] arrivals, returned to 0
+};
+
 struct ScanStepArgs {
-    const int32_t *unit_feat;   // per scan unit, UNIT_FEATS numerical features (segment order), -1 for padding
-    const uint32_t *unit_segl;  // per scan unit, its lanes a feature: 64, 16 or 4
-    uint32_t nseg;              // the units of several features come first
-    const uint32_t *cat_feats;  // the categorical features (k_step_cat)
-    uint32_t ncat;
+    const int32_t *wide_feats;  // the two-byte features
     StepPlan *plan;
 };
 
@@ -4539,23 +4639,16 @@ struct SelectArgs {
 struct ReduceStepArgs {
     const int32_t *partial;     // the step partial buffer
     const uint32_t *fmt;        // the partials' formats (per slab, per k_step_rows workgroup: 1 packed, 0 pairs)
-    const ColGroup *cgs;        // [ncg]
+    const ColGroup *cgs;        // [ncgw], the two-byte slabs'
     StepPlan *plan;
-    const uint32_t *slot_flat;  // dense slabs: per slot, its flat-histogram bin + 1 (0: none)
 };
 
-// The end of job j, by one block (learner.rs:294-352): both children's best splits from their per-feature
-// candidates (split.rs:866-880), then their leaves in the speculative tree and the job's leaf marked expanded (thread
-// 0). Up to 256 features, waves 0 and 1 take a child each while wave 2 counts the job's evaluated features; beyond,
-// half the block's waves take a child, each over a share of the features, and their bests are merged (the (gain,
-// feature) order is total, so any split of the features gives the same winner), every wave counting a share of the
-// evaluated features: one wave a child took 2000 features in 32 rounds of dependent loads, and the merge's extra
-// barrier costs small feature counts 1 us a step.
+// The end of job j, by one block (learner.rs:294-352): both children's best splits (split.rs:866-880) from their
+// candidate slots' gains, a wave a child, while the other waves count the job's evaluated features; then their leaves in
+// the speculative tree and the job's leaf marked expanded (thread 0).
 __device__ void job_select(const GrowState &g, const JobPlan &J, uint32_t j) {
     __shared__ SplitOut s_out[2];
-    __shared__ uint32_t s_used;
-    __shared__ double s_wb[2][8];
-    __shared__ int s_wf[2][8];
+    __shared__ uint32_t s_used[16];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     GrowCtl *ctl = g.ctl;
     const int64_t left = static_cast<int64_t>(J.left);
@@ -4574,96 +4667,45 @@ __device__ void job_select(const GrowState &g, const JobPlan &J, uint32_t j) {
     const int64_t min_pair = 2 * g.cfg.min_data_in_leaf;
     const bool searched = J.hist && depth_allows(g, depth) && (left >= min_pair || right >= min_pair);
     const uint32_t nw = blockDim.x >> 6;
-    if (g.nf <= 256u || nw < 4u) {  // uniform
-        // waves 0 and 1: the best split of the left and the right child; wave 2: the job's evaluated features
-        // (learner.rs:262-265), for the byte count
-        if (wave == 2) {
-            const uint8_t *prow = g.splittable + static_cast<size_t>(J.t) * g.nf;
-            uint32_t used = 0;
-            for (uint32_t f = lane; f < g.nf; f += 64u)
-                used += static_cast<uint32_t>(__popcll(__ballot(g.mask[f] != 0 && prow[f] != 0)));
-            if (lane == 0) s_used = used;
-        } else if (wave < 2) {
-            const uint32_t ch = wave;
-            SplitOut out = {};
-            if (searched) {
-                const FeatCand *cands = g.cands + (static_cast<size_t>(j) * 2 + ch) * g.nf;
-                uint8_t *row = g.splittable + static_cast<size_t>(kid + static_cast<int32_t>(ch)) * g.nf;
-                double best = 0.0;
-                int bf = -1;
-                for (uint32_t f = lane; f < g.nf; f += 64u) {
-                    const FeatCand &c = cands[f];
-                    row[f] = static_cast<uint8_t>(c.splittable);
-                    if (!c.found) continue;
-                    const double gv = (c.gain != c.gain) ? -__builtin_inf() : c.gain;
-                    if (cand_better(gv, static_cast<int>(f), best, bf)) {
-                        best = gv;
-                        bf = static_cast<int>(f);
-                    }
-                }
-                wave_best(best, bf);
-                if (bf >= 0) {  // the winner, read once more where the scans left it
-                    const int64_t cnt = ch == 0 ? left : right;
-                    out = split_out(cands[bf], bf, make_ctx(g.cfg, grow_sg(g), grow_sh(g), J.child_ug[ch], J.child_uh[ch], cnt), g.cfg);
-                }
-            }
-            if (lane == 0) s_out[ch] = out;
+    // waves 0 and 1: the best split of the left and the right child; the others: the job's evaluated features
+    // (learner.rs:262-265), for the byte count
+    if (wave >= 2) {
+        const uint8_t *prow = g.splittable + static_cast<size_t>(J.t) * g.nf;
+        uint32_t used = 0;
+        for (uint32_t f0 = (wave - 2u) * 64u; f0 < g.nf; f0 += 64u * (nw - 2u)) {
+            const uint32_t f = f0 + lane;
+            used += static_cast<uint32_t>(__popcll(__ballot(f < g.nf && g.mask[f] != 0 && prow[f] != 0)));
         }
-        __syncthreads();
+        if (lane == 0) s_used[wave] = used;
     } else {
-        // the job's evaluated features (learner.rs:262-265), for the byte count, a share a wave
-        const uint32_t wpc = nw >> 1 < 8u ? nw >> 1 : 8u;  // waves a child
-        if (threadIdx.x == 0) s_used = 0;
-        __syncthreads();
-        {
-            const uint8_t *prow = g.splittable + static_cast<size_t>(J.t) * g.nf;
-            uint32_t used = 0;
-            for (uint32_t f = threadIdx.x; f < g.nf; f += blockDim.x) used += g.mask[f] != 0 && prow[f] != 0 ? 1u : 0u;
-            used = wave_total(used);
-            if (lane == 0 && used) atomicAdd(&s_used, used);
-        }
-        // waves c wpc .. c wpc + wpc - 1: child c's best over features sub 64 + lane, + 64 wpc, ...
-        if (wave < 2u * wpc && searched) {
-            const uint32_t ch = wave / wpc, sub = wave - ch * wpc;
-            const FeatCand *cands = g.cands + (static_cast<size_t>(j) * 2 + ch) * g.nf;
-            uint8_t *row = g.splittable + static_cast<size_t>(kid + static_cast<int32_t>(ch)) * g.nf;
+        const uint32_t ch = wave;
+        SplitOut out = {};
+        if (searched) {
+            const size_t base = (static_cast<size_t>(j) * 2 + ch) * g.nslot;
             double best = 0.0;
             int bf = -1;
-            for (uint32_t f = sub * 64u + lane; f < g.nf; f += 64u * wpc) {
-                const FeatCand &c = cands[f];
-                row[f] = static_cast<uint8_t>(c.splittable);
-                if (!c.found) continue;
-                const double gv = (c.gain != c.gain) ? -__builtin_inf() : c.gain;
-                if (cand_better(gv, static_cast<int>(f), best, bf)) {
+            uint32_t bs = 0;
+            for (uint32_t s = lane; s < g.nslot; s += 64u) {
+                const double gv = g.cand_gain[base + s];
+                const int fv = g.cand_feat[base + s];
+                if (cand_better(gv, fv, best, bf)) {
                     best = gv;
-                    bf = static_cast<int>(f);
+                    bf = fv;
+                    bs = s;
                 }
             }
-            wave_best(best, bf);
-            if (lane == 0) {
-                s_wb[ch][sub] = best;
-                s_wf[ch][sub] = bf;
+            int wf = bf;
+            wave_best(best, wf);
+            if (wf >= 0) {  // the winner, read where the scans left it (a feature is in one slot)
+                const uint32_t owner = static_cast<uint32_t>(__builtin_ctzll(__ballot(bf == wf)));
+                const uint32_t slot = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bs), owner));
+                const int64_t cnt = ch == 0 ? left : right;
+                out = split_out(g.cands[base + slot], wf, make_ctx(g.cfg, grow_sg(g), grow_sh(g), J.child_ug[ch], J.child_uh[ch], cnt), g.cfg);
             }
         }
-        __syncthreads();
-        // waves 0 and 1: the left and the right child's winner over its waves' bests
-        if (wave < 2) {
-            const uint32_t ch = wave;
-            SplitOut out = {};
-            if (searched) {
-                double wb = lane < wpc ? s_wb[ch][lane] : 0.0;
-                int wf = lane < wpc ? s_wf[ch][lane] : -1;
-                wave_best(wb, wf);
-                if (wf >= 0) {  // the winner, read once more where the scans left it
-                    const FeatCand *cands = g.cands + (static_cast<size_t>(j) * 2 + ch) * g.nf;
-                    const int64_t cnt = ch == 0 ? left : right;
-                    out = split_out(cands[wf], wf, make_ctx(g.cfg, grow_sg(g), grow_sh(g), J.child_ug[ch], J.child_uh[ch], cnt), g.cfg);
-                }
-            }
-            if (lane == 0) s_out[ch] = out;
-        }
-        __syncthreads();
+        if (lane == 0) s_out[ch] = out;
     }
+    __syncthreads();
     // the children's best splits, copied a dword a thread (no child-sized copy through one thread's stack)
     static_assert(sizeof(SplitOut) % 4 == 0 && sizeof(SplitOut) / 4 <= 64, "a split copies in one wave");
     if (threadIdx.x < 128) {
@@ -4705,38 +4747,296 @@ __device__ void job_select(const GrowState &g, const JobPlan &J, uint32_t j) {
         if (J.hist) {  // the built child's histogram was made, searched or not
             const double built_rows = J.built_side == 0 ? static_cast<double>(left) : static_cast<double>(right);
             atomicAdd(&ctl->hist_rows, built_rows);
-            atomicAdd(&ctl->hist_bins, built_rows * static_cast<double>(s_used));
+            uint32_t used = 0;
+            for (uint32_t w = 2; w < nw; ++w) used += s_used[w];
+            atomicAdd(&ctl->hist_bins, built_rows * static_cast<double>(used));
             atomicAdd(&ctl->hist_builds, 1.0);
         }
         atomicAdd(&ctl->part_rows, static_cast<double>(J.count));
     }
 }
 
-// The built child's histogram of each job from its workgroups' partials, and its sibling's by subtraction in place
-// of the parent's (learner.rs:356-371). Work items (job, column group, bin range) in a grid-stride loop: a thread
-// adds one stripe of the workgroups' partials of one bin of the group's four columns, reading each partial in its
-// own format (packed: one 16-byte load; {g, h} pairs: two), and the stripes meet in LDS. grid: any, 256 threads.
-// One child's candidate of numerical feature sf in job j (split.rs:584-620), on one wave: the feature scanned in both
-// directions over the child's histogram (the built one, or the sibling the reduce formed in the parent's slot).
-template <bool WIDE>
-__device__ __forceinline__ void scan_child(const GrowState &g, const JobPlan &J, uint32_t j, int32_t sf, const FeatDev &sm,
-                                           uint32_t child) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const bool sev = g.mask[sf] != 0 && g.splittable[static_cast<size_t>(J.t) * g.nf + sf] != 0;
-    const int64_t *hist = g.pool + static_cast<size_t>(child == J.built_side ? J.built_slot : J.parent_slot) * g.slot_stride;
-    const int64_t cnt = child == 0 ? static_cast<int64_t>(J.left) : J.parent_count - static_cast<int64_t>(J.left);
-    const Ctx c = make_ctx(g.cfg, grow_sg(g), grow_sh(g), J.child_ug[child], J.child_uh[child], cnt);
-    FeatCand r = {};
-    if (scan_searched(c, sm, sev)) {
-        Grown rg = {}, fg = {};
-        bool rf, ff;
-        if constexpr (WIDE) scan_numerical_wide(c, g.cfg, sm, hist, rf, rg, ff, fg);
-        else scan_numerical(c, g.cfg, sm, hist, rf, rg, ff, fg);
-        r = feature_candidate(c, sm, rf, rg, ff, fg);
+// The children's histograms and candidates of each job over its byte slabs, one work item per (job, column group): the
+// built child's histogram of the group's four columns from the job's partials and its sibling's by subtraction in place
+// of the parent's (learner.rs:356-371), both kept in LDS, then every feature of the group scanned in both children
+// (split.rs:584-620, 694-844) from there, a wave a scan unit and child, and the group's best candidate of each child
+// written. Reducing and scanning in one launch saves the second one's start (a launch, the plan, then each scan's
+// dependent loads of a histogram another XCD just wrote): k_step_reduce 6.5 us + k_step_scan 13.7 us a step on 100k x 28
+// are 11.7 us here; 22.7 + 37.5 us in the 32-job steps of 10M x 128 are 38 us.
+// Threads: bin tid % 256, stripe tid / 256 of the partials (two stripes that meet in LDS, each then finishing two of the
+// four columns), 8 partials' loads in flight a thread. One item a block, its job found by the item's index (ChildJob):
+// with a loop over items every load of the plan came after some store, so all went through vector registers, and the
+// kernel spilled. SEG: some units hold several features; CAT: some a categorical one (apart for the registers of the plain
+// scan: two blocks a compute unit need at most 128). grid: the most items a step can have, 512 threads.
+// The sums of one bin of four columns over N partials w, w + step, ... below `groups`, their loads in flight together.
+// add_packed: packed partials. add_pairs: {g, h} pairs (PAIRS: the slab has no others), or, format by format, a mix.
+template <uint32_t N>
+__device__ __forceinline__ void add_packed(const int4 *src, size_t stride4, uint32_t w, uint32_t step, uint32_t groups, int64_t (&sg)[4],
+                                           int64_t (&sh)[4]) {
+    int4 x[N];
+#pragma unroll
+    for (uint32_t k = 0; k < N; ++k) {
+        const uint32_t wk = w + step * k;
+        x[k] = src[static_cast<size_t>(wk < groups ? wk : w) * stride4];
     }
-    if (lane == 0) g.cands[(static_cast<size_t>(j) * 2 + child) * g.nf + sf] = r;
+#pragma unroll
+    for (uint32_t k = 0; k < N; ++k) {
+        if (w + step * k >= groups) continue;
+        const int32_t v4[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int32_t gq = packed_g(v4[c]);
+            sg[c] += gq;
+            sh[c] += packed_h(v4[c], gq);
+        }
+    }
+}
+template <uint32_t N, bool PAIRS>
+__device__ __forceinline__ void add_pairs(const int4 *src, size_t stride4, size_t plane, const uint32_t *fmt, uint32_t w,
+                                          uint32_t step, uint32_t groups, int64_t (&sg)[4], int64_t (&sh)[4]) {
+    int4 a0[N], a1[N];
+    bool pk[N];
+#pragma unroll
+    for (uint32_t k = 0; k < N; ++k) {
+        const uint32_t wk = w + step * k;
+        pk[k] = !PAIRS && fmt[wk < groups ? wk : w] != 0u;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < N; ++k) {
+        const uint32_t wk = w + step * k;
+        const int4 *p = src + static_cast<size_t>(wk < groups ? wk : w) * stride4;
+        a0[k] = p[0];
+        a1[k] = p[pk[k] ? 0 : plane];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < N; ++k) {
+        if (w + step * k >= groups) continue;
+        if (pk[k]) {
+            const int32_t v4[4] = {a0[k].x, a0[k].y, a0[k].z, a0[k].w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int32_t gq = packed_g(v4[c]);
+                sg[c] += gq;
+                sh[c] += packed_h(v4[c], gq);
+            }
+        } else {
+            sg[0] += a0[k].x;
+            sg[1] += a0[k].y;
+            sg[2] += a0[k].z;
+            sg[3] += a0[k].w;
+            sh[0] += a1[k].x;
+            sh[1] += a1[k].y;
+            sh[2] += a1[k].z;
+            sh[3] += a1[k].w;
+        }
+    }
 }
 
+template <bool SEG, bool CAT>
+__global__ __launch_bounds__(512, 4) void k_step_children(GrowState g, ChildArgs a) {
+    __shared__ double plane_g[2][4 * 256], plane_h[2][4 * 256];  // [built, sibling][column * 256 + bin]
+    __shared__ int64_t red[4][512];                              // the two columns a stripe hands to the other
+    __shared__ FeatCand s_cand[8];                               // each wave's best candidate
+    __shared__ double s_gain[8];
+    __shared__ int32_t s_feat[8];
+    __shared__ __align__(16) uint8_t s_cats[CAT ? 8 * sizeof(CatScratch) : 16];
+    const StepPlan &P = *a.plan;  // empty once the tree is done (k_step_select)
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // one item a block: nothing is stored before the plan is read, so its loads are scalar ones
+    const uint32_t item = blockIdx.x, total = P.total_child;
+    const uint32_t k = item / g.ncgb, r = item - k * g.ncgb;  // the share and its item
+    uint32_t cgi = r;
+    if ((g.ncgb & 15u) == 0u) {
+        // column groups 2p and 2p + 1 (one 128-byte line of a packed partial) 8 items apart, so on one XCD (blocks
+        // go to the 8 XCDs in turn): the second reads the line from that XCD's L2
+        const uint32_t w = r & 15u;
+        cgi = 2u * ((r >> 4) * 8u + (w & 7u)) + (w >> 3);
+    }
+    const ChildJob &J = P.child[k < CHILD_MAX ? k : 0u];
+    const ColGroup &cg = a.cgs[cgi];  // read in place: a column is picked per thread
+    // wave w scans units w / 2, w / 2 + 4, ... of child w % 2: its first unit's record comes with the job
+    const uint32_t child = wave & 1u, units = SEG ? cg.unit_count : CG_COLS;
+    const uint32_t first = SEG ? cg.unit_first : CG_COLS * cgi;
+    uint32_t segl = 64u;
+    UnitRec rec;
+    auto load_rec = [&](uint32_t u) {
+        if constexpr (SEG) {
+            segl = a.unit_segl[first + u];  // wave-uniform
+            rec = a.recs[static_cast<size_t>(first + u) * UNIT_FEATS + lane / segl];
+        } else {
+            rec = a.recs[first + u];
+        }
+    };
+    if (item >= total) return;
+    if (wave >> 1 < units) load_rec(wave >> 1);
+    else rec = UnitRec{-1, 0u, FeatDev{}};
+    const uint32_t left = P.jobs[J.j].left, mixed = P.pairs[J.j];
+    const uint8_t *prow = g.splittable + static_cast<size_t>(J.t) * g.nf;
+    bool sev = rec.feat >= 0 && g.mask[rec.feat] != 0 && prow[rec.feat] != 0;
+    int64_t *built = g.pool + static_cast<size_t>(J.built_slot) * g.slot_stride;
+    int64_t *parent = g.pool + static_cast<size_t>(J.parent_slot) * g.slot_stride;
+    {
+        const size_t stride4 = step_partial_stride(cg.width) / 2;  // int4s from one partial to the next
+        const uint32_t q = wave >> 2, bin = tid & 255u;            // this thread's stripe (wave-uniform) and bin
+        // bin `bin` of the group's columns in a partial: int4 (bin / 4) * W + c0 + bin % 4, of packed words or, in a
+        // partial of pairs, of its g plane, the h plane's 64 W int4s on
+        const int4 *src = reinterpret_cast<const int4 *>(a.partial + 2 * cg.partial) + static_cast<size_t>(J.group_base) * stride4 +
+                          static_cast<size_t>(bin / 4u) * cg.width + cg.c0 + bin % 4u;
+        const size_t plane = 64u * static_cast<size_t>(cg.width);
+        const uint32_t *fmt = a.fmt + cg.fmt + J.group_base;
+        // this thread finishes columns 2q and 2q + 1: their slots' flat bins + 1 (0: none) and the parent's units,
+        // loaded with the partials
+        const uint32_t seg = bin >> cg.seg_shift, vb = bin & ((1u << cg.seg_shift) - 1u);
+        uint32_t fl[2];
+        if (cg.dense) {
+            const uint2 t = *reinterpret_cast<const uint2 *>(a.slot_flat + cg.slot_base + static_cast<size_t>(bin) * cg.width + cg.c0 + 2u * q);
+            fl[0] = t.x;
+            fl[1] = t.y;
+        } else {
+#pragma unroll
+            for (uint32_t c = 0; c < 2; ++c)
+                fl[c] = vb < cg.bins[seg][2u * q + c] ? cg.offset[seg][2u * q + c] + vb + 1u : 0u;
+        }
+        longlong2 par[2];
+#pragma unroll
+        for (uint32_t c = 0; c < 2; ++c)
+            par[c] = *reinterpret_cast<const longlong2 *>(parent + 2 * static_cast<size_t>(fl[c] ? fl[c] - 1u : 0u));
+        int64_t sg[4] = {0, 0, 0, 0}, sh[4] = {0, 0, 0, 0};
+        if (cg.pairs) {
+            for (uint32_t w = q; w < J.groups; w += 16u) add_pairs<8, true>(src, stride4, plane, fmt, w, 2u, J.groups, sg, sh);
+        } else if (mixed) {
+            for (uint32_t w = q; w < J.groups; w += 16u) add_pairs<8, false>(src, stride4, plane, fmt, w, 2u, J.groups, sg, sh);
+        } else {
+            uint32_t w = q;
+            for (; w + 2u < J.groups; w += 16u) add_packed<8>(src, stride4, w, 2u, J.groups, sg, sh);
+            if (w < J.groups) add_packed<1>(src, stride4, w, 2u, J.groups, sg, sh);
+        }
+        int64_t mg[2], mh[2];
+        const uint32_t to = q * 256u + bin, from = (1u - q) * 256u + bin;
+#pragma unroll
+        for (uint32_t c = 0; c < 2; ++c) {
+            red[2 * c][to] = q == 0u ? sg[2 + c] : sg[c];
+            red[2 * c + 1][to] = q == 0u ? sh[2 + c] : sh[c];
+            mg[c] = q == 0u ? sg[c] : sg[2 + c];
+            mh[c] = q == 0u ? sh[c] : sh[2 + c];
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t c = 0; c < 2; ++c) {
+            mg[c] += red[2 * c][from];
+            mh[c] += red[2 * c + 1][from];
+        }
+        if (J.ways > 1u) {  // the last of the job's shares to arrive adds them all up and goes on (exact integers)
+            int64_t *mine = a.scratch + ((static_cast<size_t>(J.scratch) + J.way) * g.ncgb + cgi) * 2048 + tid;
+#pragma unroll
+            for (uint32_t c = 0; c < 2; ++c) {
+                mine[(2 * c) * 512] = mg[c];
+                mine[(2 * c + 1) * 512] = mh[c];
+            }
+            if (!arrive_last(a.counters + static_cast<size_t>(J.scratch) * g.ncgb + cgi, J.ways)) return;
+            const int64_t *all = a.scratch + (static_cast<size_t>(J.scratch) * g.ncgb + cgi) * 2048 + tid;
+            for (uint32_t w = 0; w < J.ways; ++w) {
+                if (w == J.way) continue;
+                const int64_t *o = all + static_cast<size_t>(w) * g.ncgb * 2048;
+#pragma unroll
+                for (uint32_t c = 0; c < 2; ++c) {
+                    mg[c] += o[(2 * c) * 512];
+                    mh[c] += o[(2 * c + 1) * 512];
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < 2; ++c) {
+            const uint32_t at = (2u * q + c) * 256u + bin;
+            const int64_t og = par[c].x - mg[c], oh = par[c].y - mh[c];
+            plane_g[0][at] = static_cast<double>(mg[c]);
+            plane_h[0][at] = static_cast<double>(mh[c]);
+            plane_g[1][at] = static_cast<double>(og);
+            plane_h[1][at] = static_cast<double>(oh);
+            if (fl[c]) {
+                const size_t o = 2 * static_cast<size_t>(fl[c] - 1u);
+                *reinterpret_cast<longlong2 *>(built + o) = make_longlong2(mg[c], mh[c]);
+                *reinterpret_cast<longlong2 *>(parent + o) = make_longlong2(og, oh);
+            }
+        }
+    }
+    const uint32_t which = child == J.built_side ? 0u : 1u;
+    const int64_t cnt = child == 0 ? static_cast<int64_t>(left) : J.parent_count - static_cast<int64_t>(left);
+    const Ctx c = make_ctx(g.cfg, grow_sg(g), grow_sh(g), child ? J.child_ug[1] : J.child_ug[0],
+                           child ? J.child_uh[1] : J.child_uh[0], cnt);
+    uint8_t *row = g.splittable + static_cast<size_t>(J.kid + static_cast<int32_t>(child)) * g.nf;
+    __syncthreads();
+    double best = 0.0;
+    int bf = -1;
+    for (uint32_t u = wave >> 1; u < units; u += 4u) {
+        if (u >= 4u) {
+            load_rec(u);
+            sev = rec.feat >= 0 && g.mask[rec.feat] != 0 && prow[rec.feat] != 0;
+        }
+        const LdsUnits h{&plane_g[which][rec.at], &plane_h[which][rec.at]};
+        FeatCand cand = {};
+        bool rf = false, ff = false;
+        Grown rg = {}, fg = {};
+        const bool on = scan_searched(c, rec.m, sev);
+        if (CAT && segl == 64u && rec.m.kind == 2) {
+            if (on) cand = categorical_candidate(c, g.cfg, rec.m, h, reinterpret_cast<CatScratch *>(s_cats)[wave], nullptr);
+        } else {
+            if (segl == 64u) {
+                if (on) scan_numerical<64>(c, g.cfg, rec.m, h, rf, rg, ff, fg);
+            } else if (SEG) {
+                if (segl == 16u) scan_numerical<16>(c, g.cfg, rec.m, h, rf, rg, ff, fg);
+                else scan_numerical<4>(c, g.cfg, rec.m, h, rf, rg, ff, fg);
+            }
+            if (on) cand = feature_candidate(c, rec.m, rf, rg, ff, fg);
+        }
+        const bool lead = rec.feat >= 0 && (lane & (segl - 1u)) == 0u;
+        if (lead) row[rec.feat] = static_cast<uint8_t>(cand.splittable);
+        // the unit's best by (gain, lower feature), against the wave's so far
+        double wg = lead && cand.found ? (cand.gain != cand.gain ? -__builtin_inf() : cand.gain) : 0.0;
+        int wf = lead && cand.found ? rec.feat : -1;
+        const int mine = wf;
+        if (SEG && segl != 64u) {
+            wave_best(wg, wf);
+        } else {
+            wg = readlane_f64(wg, 0);
+            wf = __builtin_amdgcn_readlane(wf, 0);
+        }
+        if (cand_better(wg, wf, best, bf)) {
+            best = wg;
+            bf = wf;
+            if (mine == wf) s_cand[wave] = cand;
+        }
+    }
+    if (lane == 0) {
+        s_gain[wave] = best;
+        s_feat[wave] = bf;
+    }
+    __syncthreads();
+    if (wave < 2) {  // child `wave`'s best over its four waves
+        double wg = lane < 4 ? s_gain[wave + 2 * lane] : 0.0;
+        int wf = lane < 4 ? s_feat[wave + 2 * lane] : -1;
+        const int mine = wf;
+        wave_best(wg, wf);
+        const size_t slot = (static_cast<size_t>(J.j) * 2 + wave) * g.nslot + cgi;
+        if (lane == 0) {
+            g.cand_gain[slot] = wg;
+            g.cand_feat[slot] = wf;
+        }
+        static_assert(sizeof(FeatCand) % 4 == 0 && sizeof(FeatCand) / 4 <= 64, "a candidate copies in one wave");
+        if (wf >= 0) {
+            const uint32_t owner = wave + 2u * static_cast<uint32_t>(__builtin_ctzll(__ballot(mine == wf)));
+            if (lane < sizeof(FeatCand) / 4)
+                reinterpret_cast<uint32_t *>(&g.cands[slot])[lane] = reinterpret_cast<const uint32_t *>(&s_cand[owner])[lane];
+        }
+    }
+}
+
+// The two-byte slabs' histograms of each job: the built child's from its workgroups' partials, and its sibling's by
+// subtraction in place of the parent's (learner.rs:356-371). Work items (job, column group, bin range) in a grid-stride
+// loop: a thread adds one stripe of the workgroups' partials of one bin of the group's four columns, reading each partial
+// in its own format (packed: one 16-byte load; {g, h} pairs: two), and the stripes meet in LDS. (A two-byte feature's
+// bins lie in four column groups, so its scan is a launch of its own.) grid: any, 256 threads.
 __global__ __launch_bounds__(256) void k_step_reduce(GrowState g, ReduceStepArgs a) {
     __shared__ int64_t red[8][256];  // the stripes' sums, [value][thread]: conflict-free
     const StepPlan &P = *a.plan;  // empty once the tree is done (k_step_select)
@@ -4747,7 +5047,7 @@ __global__ __launch_bounds__(256) void k_step_reduce(GrowState g, ReduceStepArgs
         const uint32_t ways = J.ways, groups = J.groups;
         const uint32_t r = item - J.red_base;
         uint32_t cgi, sub;
-        if ((g.ncg & 15u) == 0u) {
+        if ((g.ncgw & 15u) == 0u) {
             // column groups 2p and 2p + 1 (one 128-byte line of a packed partial) 8 items apart, so on one XCD (blocks
             // go to the 8 XCDs in turn): the second reads the line from that XCD's L2
             const uint32_t w = r & 15u, pi = (r >> 4) * 8u + (w & 7u), pair = pi / ways;
@@ -4764,27 +5064,18 @@ __global__ __launch_bounds__(256) void k_step_reduce(GrowState g, ReduceStepArgs
         const uint32_t ns = 256u / ways;                           // the item's bins
         const uint32_t q = tid / ns;                               // this thread's stripe
         const uint32_t bin = sub * ns + tid % ns;
-        // bin `bin` of the group's columns in a partial: packed, int4 (bin / 4) * W + c0 + bin % 4; pairs, the int4s
-        // at (bin * W + c0) / 2 and the next
-        const int4 *src = reinterpret_cast<const int4 *>(a.partial + 2 * cg.partial) + static_cast<size_t>(J.group_base) * stride4;
-        const size_t po = static_cast<size_t>(bin / 4u) * cg.width + cg.c0 + bin % 4u;
-        const size_t qo = (static_cast<size_t>(bin) * cg.width + cg.c0) / 2;
+        // bin `bin` of the group's columns in a partial: int4 (bin / 4) * W + c0 + bin % 4, of packed words or, in a
+        // partial of pairs, of its g plane, the h plane's 64 W int4s on
+        const int4 *src = reinterpret_cast<const int4 *>(a.partial + 2 * cg.partial) + static_cast<size_t>(J.group_base) * stride4 +
+                          static_cast<size_t>(bin / 4u) * cg.width + cg.c0 + bin % 4u;
+        const size_t plane = 64u * static_cast<size_t>(cg.width);
         const uint32_t *fmt = a.fmt + cg.fmt + J.group_base;
         // the parent's bins are loaded with the partials (the writes below need them); every partial is first read
         // as packed, and a {g, h} pair partial (a workgroup that flushed) is read again in its own layout
-        const uint32_t seg = bin >> cg.seg_shift, vb = bin & ((1u << cg.seg_shift) - 1u);
         // the flat bin + 1 of each of the four columns' slot (0: none)
         uint32_t fl[4];
-        if (cg.dense) {
-            const uint4 t = *reinterpret_cast<const uint4 *>(a.slot_flat + cg.slot_base + static_cast<size_t>(bin) * cg.width + cg.c0);
-            fl[0] = t.x;
-            fl[1] = t.y;
-            fl[2] = t.z;
-            fl[3] = t.w;
-        } else {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) fl[c] = vb < cg.bins[seg][c] ? cg.offset[seg][c] + vb * cg.stride[c] + 1u : 0u;
-        }
+        for (int c = 0; c < 4; ++c) fl[c] = bin < cg.bins[0][c] ? cg.offset[0][c] + bin * cg.stride[c] + 1u : 0u;
         int64_t pg[4] = {0, 0, 0, 0}, ph[4] = {0, 0, 0, 0};
         if (q == 0) {
 #pragma unroll
@@ -4798,40 +5089,9 @@ __global__ __launch_bounds__(256) void k_step_reduce(GrowState g, ReduceStepArgs
         }
         int64_t sg[4] = {0, 0, 0, 0}, sh[4] = {0, 0, 0, 0};
         for (uint32_t w = q; w < groups; w += 8u * ways) {
-            bool pk[8];
-            int4 x[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const uint32_t wk = w + k * ways;
-                const uint32_t wc = wk < groups ? wk : q;
-                pk[k] = fmt[wc] != 0u;
-                x[k] = src[static_cast<size_t>(wc) * stride4 + po];
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const uint32_t wk = w + k * ways;
-                if (wk >= groups) continue;
-                if (pk[k]) {
-                    const int32_t v4[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const int32_t gq = packed_g(v4[c]);
-                        sg[c] += gq;
-                        sh[c] += packed_h(v4[c], gq);
-                    }
-                } else {
-                    const int4 *p = src + static_cast<size_t>(wk) * stride4;
-                    const int4 a0 = p[qo], a1 = p[qo + 1];
-                    sg[0] += a0.x;
-                    sh[0] += a0.y;
-                    sg[1] += a0.z;
-                    sh[1] += a0.w;
-                    sg[2] += a1.x;
-                    sh[2] += a1.y;
-                    sg[3] += a1.z;
-                    sh[3] += a1.w;
-                }
-            }
+            if (cg.pairs) add_pairs<8, true>(src, stride4, plane, fmt, w, ways, groups, sg, sh);
+            else if (P.pairs[j]) add_pairs<8, false>(src, stride4, plane, fmt, w, ways, groups, sg, sh);
+            else add_packed<8>(src, stride4, w, ways, groups, sg, sh);
         }
         if (ways > 1u) {
 #pragma unroll
@@ -4865,78 +5125,38 @@ __global__ __launch_bounds__(256) void k_step_reduce(GrowState g, ReduceStepArgs
     }
 }
 
-// Scan items (job, unit, child), a wave each in a grid-stride loop: the unit's numerical feature scanned in both
-// directions (split.rs:584-620) and its candidate written. Categorical features are k_step_cat's; features of
-// two-byte bins are k_step_scan<true>'s, the others k_step_scan<false>'s. grid: any, 256 threads.
-template <bool WIDE>
-__global__ __launch_bounds__(256, WIDE ? 1 : 4) void k_step_scan(GrowState g, ScanStepArgs a) {
+// Scan items (job, two-byte feature, child), a wave each in a grid-stride loop: the feature scanned in both directions
+// (split.rs:584-620) over the child's histogram (the built one, or the sibling k_step_reduce formed in the parent's slot)
+// and its candidate written to its own slot. grid: any, 256 threads.
+__global__ __launch_bounds__(256) void k_step_scan(GrowState g, ScanStepArgs a) {
     const StepPlan &P = *a.plan;  // empty once the tree is done (k_step_select)
-    const uint32_t total = P.total_scan * 2u;  // scan items count units: a wave per unit and child
-    for (uint32_t item = blockIdx.x * 4u + (threadIdx.x >> 6); item < total; item += gridDim.x * 4u) {
-        const uint32_t gi = item >> 1, child = item & 1u;
-        const uint32_t j = job_of(P.scan_base, P.njobs, gi);
-        const JobPlan &J = P.jobs[j];
-        const uint32_t u = gi - J.scan_base;
-        if (u < a.nseg) continue;  // k_step_scan_seg's
-        const int32_t sf = a.unit_feat[u * UNIT_FEATS];
-        if (sf < 0) continue;
-        const FeatDev sm = g.feats[sf];
-        if (sm.kind == 2 || (sm.wide != 0) != WIDE) continue;  // the other instantiation's, or k_step_cat's
-        scan_child<WIDE>(g, J, j, sf, sm, child);
-    }
-}
-
-// The scan units of several byte features a wave (k_step_scan's items of 16 or 4 lanes a feature): every segment
-// scans (its shuffles take the whole wave), a padding or unsearched one keeping nothing. Its own kernel, so that the
-// wave-wide scan keeps its registers (and occupancy). grid: any, 256 threads.
-__global__ __launch_bounds__(256) void k_step_scan_seg(GrowState g, ScanStepArgs a) {
-    const StepPlan &P = *a.plan;
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t total = P.total_scan * 2u;
+    const uint32_t total = P.total_scan * 2u;  // scan items count features: a wave per feature and child
     for (uint32_t item = blockIdx.x * 4u + (threadIdx.x >> 6); item < total; item += gridDim.x * 4u) {
         const uint32_t gi = item >> 1, child = item & 1u;
         const uint32_t j = job_of(P.scan_base, P.njobs, gi);
         const JobPlan &J = P.jobs[j];
         const uint32_t u = gi - J.scan_base;
-        if (u >= a.nseg) continue;  // k_step_scan's
-        const uint32_t segl = a.unit_segl[u];  // 16 or 4, wave-uniform
-        const uint32_t t = lane & (segl - 1u);
-        const int32_t sf = a.unit_feat[u * UNIT_FEATS + lane / segl];
-        const FeatDev sm = sf >= 0 ? g.feats[sf] : FeatDev{};
-        const bool sev = sf >= 0 && g.mask[sf] != 0 && g.splittable[static_cast<size_t>(J.t) * g.nf + sf] != 0;
+        const int32_t sf = a.wide_feats[u];
+        const FeatDev sm = g.feats[sf];
+        const bool sev = g.mask[sf] != 0 && g.splittable[static_cast<size_t>(J.t) * g.nf + sf] != 0;
         const int64_t *hist = g.pool + static_cast<size_t>(child == J.built_side ? J.built_slot : J.parent_slot) * g.slot_stride;
         const int64_t cnt = child == 0 ? static_cast<int64_t>(J.left) : J.parent_count - static_cast<int64_t>(J.left);
         const Ctx c = make_ctx(g.cfg, grow_sg(g), grow_sh(g), J.child_ug[child], J.child_uh[child], cnt);
-        Grown rg = {}, fg = {};
-        bool rf = false, ff = false;
-        if (segl == 16u) scan_numerical<16>(c, g.cfg, sm, hist, rf, rg, ff, fg);
-        else scan_numerical<4>(c, g.cfg, sm, hist, rf, rg, ff, fg);
         FeatCand r = {};
-        if (sf >= 0 && scan_searched(c, sm, sev)) r = feature_candidate(c, sm, rf, rg, ff, fg);
-        if (t == 0 && sf >= 0) g.cands[(static_cast<size_t>(j) * 2 + child) * g.nf + sf] = r;
-    }
-}
-
-// The categorical features' candidates of every job (split.rs:694-844): a wave per (job, feature, child) in a
-// grid-stride loop. grid: any, 256 threads.
-__global__ __launch_bounds__(256) void k_step_cat(GrowState g, ScanStepArgs a) {
-    __shared__ CatScratch cats[4];
-    const StepPlan &P = *a.plan;  // empty once the tree is done (k_step_select)
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const uint32_t per_job = 2 * a.ncat, total = P.njobs * per_job;
-    for (uint32_t item = blockIdx.x * 4 + wave; item < total; item += gridDim.x * 4) {
-        const uint32_t j = item / per_job, r = item - j * per_job, child = r & 1u;
-        const JobPlan &J = P.jobs[j];
-        if (!J.hist) continue;
-        const uint32_t f = a.cat_feats[r >> 1];
-        const FeatDev sm = g.feats[f];
-        const bool sev = g.mask[f] != 0 && g.splittable[static_cast<size_t>(J.t) * g.nf + f] != 0;
-        const int64_t *hist = g.pool + static_cast<size_t>(child == J.built_side ? J.built_slot : J.parent_slot) * g.slot_stride;
-        const int64_t cnt = child == 0 ? static_cast<int64_t>(J.left) : J.parent_count - static_cast<int64_t>(J.left);
-        const Ctx c = make_ctx(g.cfg, grow_sg(g), grow_sh(g), J.child_ug[child], J.child_uh[child], cnt);
-        FeatCand out = {};
-        if (scan_searched(c, sm, sev)) out = categorical_candidate(c, g.cfg, sm, hist, cats[wave], nullptr);
-        if (lane == 0) g.cands[(static_cast<size_t>(j) * 2 + child) * g.nf + f] = out;
+        if (scan_searched(c, sm, sev)) {
+            Grown rg = {}, fg = {};
+            bool rf, ff;
+            scan_numerical_wide(c, g.cfg, sm, hist, rf, rg, ff, fg);
+            r = feature_candidate(c, sm, rf, rg, ff, fg);
+        }
+        if (lane == 0) {
+            const size_t slot = (static_cast<size_t>(j) * 2 + child) * g.nslot + g.ncgb + u;
+            g.cands[slot] = r;
+            g.cand_gain[slot] = r.gain != r.gain ? -__builtin_inf() : r.gain;
+            g.cand_feat[slot] = r.found ? sf : -1;
+            g.splittable[static_cast<size_t>(J.kid + static_cast<int32_t>(child)) * g.nf + sf] = static_cast<uint8_t>(r.splittable);
+        }
     }
 }
 
@@ -4949,6 +5169,7 @@ __global__ __launch_bounds__(512) void k_step_select(GrowState g, SelectArgs a) 
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         a.next->njobs = 0;
         a.next->total_groups = 0;
+        a.next->total_child = 0;
         a.next->total_red = 0;
         a.next->total_scan = 0;
     }
