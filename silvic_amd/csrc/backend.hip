@@ -1993,7 +1993,6 @@ struct Context {
     // split steps (k_step_rows, k_step_children, k_step_reduce, k_step_scan, k_step_select)
     DevBuf<int32_t> step_partial;            // per slab: [cus + JMAX][256 * W] {g, h}
     DevBuf<unsigned long long> tile_status;  // per partition tile
-    DevBuf<uint32_t> fin_counts;             // the jobs-selected counter of k_step_select
     DevBuf<int64_t> child_scratch;           // k_step_children: the sums of shared jobs' shares, and their arrivals
     DevBuf<uint32_t> child_counts;
     uint64_t epochs_used = 0;
@@ -2054,7 +2053,6 @@ struct Context {
         h_sums.alloc(2 * static_cast<size_t>(L));
         step_partial.alloc(2 * step_partial_pairs);
         tile_status.alloc(div_up(rows, STEP_TILE) + JMAX + 1);
-        fin_counts.alloc(1);
         reset_step_state();
         grow_capacity = L;
     }
@@ -2074,7 +2072,6 @@ struct Context {
     void reset_step_state() {
         hip_check(hipMemsetAsync(dtree.p + tree_layout.ctl, 0, sizeof(GrowCtl), stream), "zero grow control");
         hip_check(hipMemsetAsync(tile_status.p, 0, tile_status.n * sizeof(unsigned long long), stream), "zero tile status");
-        hip_check(hipMemsetAsync(fin_counts.p, 0, fin_counts.n * sizeof(uint32_t), stream), "zero step counters");
         epochs_used = 0;
     }
 
@@ -2126,6 +2123,7 @@ struct Context {
         // a workgroup's i32 sums take at most (2^31 - 1) / max_q rows
         const uint64_t mq = static_cast<uint64_t>(std::max<int64_t>(std::max(max_gq, max_hq), 1));
         g.tile_cap = static_cast<uint32_t>(std::max<uint64_t>(std::min<uint64_t>((2147483647ull / mq) / STEP_TILE, 1u << 30), 1));
+        g.count_work = prof.on ? 1u : 0u;
         g.hist_weight = STEP_HIST_WEIGHT;
         g.sparse_weight = STEP_SPARSE_WEIGHT;
         return g;
@@ -2451,9 +2449,9 @@ void Context::grow(const srocm_grow_spec &spec, HostTree &tree, std::vector<sroc
                     k_step_scan<<<scan_blocks(), 256, 0, stream>>>(g, sca);
                     launch_check("k_step_scan");
                 }
-                SelectArgs sa2{fin_counts.p, d_plans.p + parity, d_plans.p + (parity ^ 1u)};
-                if (L <= LEAVES_SMALL) k_step_select<LEAVES_SMALL><<<g.jcap, 512, 0, stream>>>(g, sa2);
-                else k_step_select<GROW_MAX_LEAVES><<<g.jcap, 512, 0, stream>>>(g, sa2);
+                SelectArgs sa2{d_plans.p + parity, d_plans.p + (parity ^ 1u)};
+                if (L <= LEAVES_SMALL) k_step_select<LEAVES_SMALL><<<1, select_threads<LEAVES_SMALL>(), 0, stream>>>(g, sa2);
+                else k_step_select<GROW_MAX_LEAVES><<<1, select_threads<GROW_MAX_LEAVES>(), 0, stream>>>(g, sa2);
                 launch_check("k_step_select");
             }
             if (after_steps) {

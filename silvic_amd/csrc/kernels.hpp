@@ -1079,6 +1079,7 @@ struct FeatCand {
     double left_units_g, left_units_h;
     uint32_t col;         // the feature's column-major index (its bins for the partition)
     uint32_t nan_idx;     // its NaN bin, or NO_BIN
+    uint32_t wide;        // it has two-byte bins (rule_left)
     uint32_t rule;        // RULE_NUMERICAL, RULE_ONEHOT or RULE_SORTED
     uint32_t cat_forward; // sorted categorical: the run went from the low end of the sorted order
     uint32_t cat_count;   // categorical: bins going left
@@ -1269,32 +1270,6 @@ __device__ __forceinline__ uint64_t wave_max_u64_hi(uint64_t v) {
                             : wave_max_u32(hi == mh ? lo : 0u);
     return (static_cast<uint64_t>(mh) << 32) | ml;
 }
-
-// A feature candidate as held by lane `owner`, broadcast to the wave.
-__device__ __forceinline__ FeatCand readlane_cand(const FeatCand &c, uint32_t owner) {
-    FeatCand r;
-    r.found = __builtin_amdgcn_readlane(c.found, owner);
-    r.splittable = __builtin_amdgcn_readlane(c.splittable, owner);
-    r.gain = readlane_f64(c.gain, owner);
-    r.best_gain = readlane_f64(c.best_gain, owner);
-    r.threshold = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c.threshold), owner));
-    r.default_left = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c.default_left), owner));
-    r.left_grad = readlane_f64(c.left_grad, owner);
-    r.left_hess = readlane_f64(c.left_hess, owner);
-    r.left_count = static_cast<int64_t>(readlane_u64(static_cast<uint64_t>(c.left_count), owner));
-    r.left_units_g = readlane_f64(c.left_units_g, owner);
-    r.left_units_h = readlane_f64(c.left_units_h, owner);
-    r.col = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c.col), owner));
-    r.nan_idx = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c.nan_idx), owner));
-    r.rule = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c.rule), owner));
-    r.cat_forward = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c.cat_forward), owner));
-    r.cat_count = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c.cat_count), owner));
-#pragma unroll
-    for (int w = 0; w < 8; ++w)
-        r.cat_mask[w] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c.cat_mask[w]), owner));
-    return r;
-}
-
 
 struct FeatDev {
     uint32_t num_bins, hist_offset, kind, nan_bin;
@@ -1786,6 +1761,7 @@ __device__ FeatCand feature_candidate(const Ctx &c, const FeatDev &m, bool rf, c
         r.gain = r.best_gain - c.min_gain_shift;
         r.col = m.col;
         r.nan_idx = m.nan_bin ? m.num_bins - 1 : NO_BIN;
+        r.wide = m.wide;
     }
     return r;
 }
@@ -2166,6 +2142,7 @@ struct SplitOut {
     double left_output, right_output;
     uint32_t col, nan_idx;  // the feature's column-major index and NaN bin (NO_BIN: none)
     uint32_t rule;          // RULE_*: categorical rules send exactly the bins of cat_mask left
+    uint32_t wide;          // the feature has two-byte bins
     uint32_t cat_count;
     uint32_t cat_mask[8];
 };
@@ -2193,6 +2170,7 @@ __device__ __forceinline__ SplitOut split_out(const FeatCand &c, int f, const Ct
     o.col = c.col;
     o.nan_idx = c.nan_idx;
     o.rule = c.rule;
+    o.wide = c.wide;
     o.cat_count = c.cat_count;
     for (int w = 0; w < 8; ++w) o.cat_mask[w] = c.cat_mask[w];
     if (c.rule != RULE_NUMERICAL) {
@@ -2302,18 +2280,21 @@ __device__ __forceinline__ uint32_t reduce_ways(uint32_t groups) {
     return w;
 }
 
-// Wave-wide sums of one value per lane: exclusive prefix and total.
+// Wave-wide sums of one value per lane (every lane active): inclusive and exclusive prefix, total. DPP steps: the plan's
+// nine prefixes on one wave took 54 dependent LDS permutes by __shfl_up.
 __device__ __forceinline__ uint32_t wave_incl_sum(uint32_t v) {
-    const uint32_t lane = threadIdx.x & 63u;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t x = __shfl_up(v, o);
-        if (lane >= static_cast<uint32_t>(o)) v += x;
-    }
+    v += dpp_u32<DPP_ROW_SHR1, 0xf>(v);
+    v += dpp_u32<DPP_ROW_SHR2, 0xf>(v);
+    v += dpp_u32<DPP_ROW_SHR4, 0xf>(v);
+    v += dpp_u32<DPP_ROW_SHR8, 0xf>(v);
+    v += dpp_u32<DPP_ROW_BCAST15, 0xa>(v);
+    v += dpp_u32<DPP_ROW_BCAST31, 0xc>(v);
     return v;
 }
 __device__ __forceinline__ uint32_t wave_excl_sum(uint32_t v) { return wave_incl_sum(v) - v; }
-__device__ __forceinline__ uint32_t wave_total(uint32_t v) { return __shfl(wave_incl_sum(v), 63); }
+__device__ __forceinline__ uint32_t wave_total(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(wave_incl_sum(v)), 63));
+}
 __device__ __forceinline__ float wave_total_f32(float v) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
@@ -2397,6 +2378,9 @@ struct JobPlan {
     int32_t kid;                  // the children's speculative leaves
     int64_t parent_count;
     double child_ug[2], child_uh[2];  // the children's sums in histogram units (left, right)
+    double child_out[2];          // their outputs
+    int32_t depth;                // and depth
+    uint32_t pad_;
 };
 
 // What k_step_children needs of a histogrammed job, found by its item's index alone (item / column groups), so that a
@@ -2500,6 +2484,7 @@ struct GrowState {
     uint32_t nslot;           // ncgb + nwide
     uint32_t flush_rows;      // rows a packed 16/16 LDS word can take
     uint32_t tile_cap;        // k_step_rows tiles a workgroup may take (its i32 sums of the quantized units)
+    uint32_t count_work;      // keep the control block's byte-count totals (hist_rows ... part_rows)
     float hist_weight;        // the planner's cost of a tile of histogrammed rows, in partitioned tiles of a dense
     float sparse_weight;      // leaf, and the most a tile of a sparse leaf costs more
 };
@@ -3159,45 +3144,30 @@ __device__ __forceinline__ void replay(S &s, uint32_t n0, uint32_t L) {
     }
 }
 
+// The `spec` highest candidate keys for a few expansions (spec <= SPEC_FEW), on one wave: `spec` rounds of a wave
+// maximum over the keys below the last one taken. The keys are distinct and end in 8191 - leaf, so round r finds the key
+// ranked r and its leaf: jobs 1 .. spec in descending key order, as the ranking orders them.
+template <typename S>
+__device__ __forceinline__ void top_few(S &s, uint32_t ncand, uint32_t spec) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t first = lane < ncand ? s.ckey[lane] : 0ull;  // the only one of a lane up to 64 candidates
+    uint64_t last = ~0ull;
+    for (uint32_t r = 0; r < spec; ++r) {
+        uint64_t best = first < last ? first : 0ull;
+        for (uint32_t i = lane + 64u; i < ncand; i += 64u) {
+            const uint64_t k = s.ckey[i];
+            best = k < last && k > best ? k : best;
+        }
+        last = wave_max_u64_hi(best);
+        if (lane == 0) s.job_t[1 + r] = static_cast<uint16_t>(8191u - (static_cast<uint32_t>(last) & 8191u));
+    }
+}
+
 // The `spec` highest of the `ncand` candidate keys s.ckey (distinct 64-bit keys) into s.job_t[1 .. spec], in key
 // order, by a radix selection over the keys' 64 bits, 8 at a time from the top: a 256-bucket count of the
 // candidates that still match the prefix found so far, the bucket where the count from the top reaches what is
 // left to take, and the candidates above it taken. Every key is distinct, so after at most 8 rounds the prefix
 // is a whole key. Block-wide; s.crank holds the counts.
-// The `spec` highest candidate keys for a few expansions (spec <= SPEC_FEW), on one wave: `spec` rounds of a wave
-// maximum over the keys not yet taken, each lane holding candidates lane, lane + 64, ... (at most 64 of them, a bit
-// each in `taken`). The keys are distinct (they end in the leaf), so round r finds the key ranked r: jobs 1 .. spec in
-// descending key order, as the ranking orders them.
-template <typename S>
-__device__ __forceinline__ void top_few(S &s, uint32_t ncand, uint32_t spec) {
-    static_assert(S::CAND <= 64u * 64u, "a lane's candidates fit the taken mask");
-    const uint32_t lane = threadIdx.x & 63u;
-    uint64_t taken = 0;
-    for (uint32_t r = 0; r < spec; ++r) {
-        uint64_t best = 0;
-        uint32_t at = 0;
-        uint32_t q = 0;
-        for (uint32_t i = lane; i < ncand; i += 64u, ++q) {
-            const uint64_t k = s.ckey[i];
-            if (!((taken >> q) & 1ull) && k > best) {
-                best = k;
-                at = i;
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            const uint64_t ob = __shfl_xor(best, o);
-            const uint32_t oa = static_cast<uint32_t>(__shfl_xor(static_cast<int>(at), o));
-            if (ob > best) {
-                best = ob;
-                at = oa;
-            }
-        }
-        // every candidate key is nonzero (a positive gain's bits), so the winner is a real candidate
-        if ((at & 63u) == lane) taken |= 1ull << (at >> 6);
-        if (lane == 0) s.job_t[1 + r] = s.cand[at];
-    }
-}
-
 template <uint32_t MAXL>
 __device__ void select_top(AdvShared<MAXL> &s, uint32_t ncand, uint32_t spec) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, nt = blockDim.x;
@@ -3279,9 +3249,8 @@ __device__ void apply_commits(const GrowState &g, const AdvShared<MAXL> &s, uint
             const SplitOut &info = p.best;
             const uint32_t node = n0 - 1 + c;
             t.split_feature[node] = info.feature;
-            const uint32_t wide = g.feats[info.feature].wide;
 #pragma unroll
-            for (uint32_t w = 0; w < 8; ++w) t.left_bins[static_cast<size_t>(node) * 8 + w] = left_bins_word(info, w, wide);
+            for (uint32_t w = 0; w < 8; ++w) t.left_bins[static_cast<size_t>(node) * 8 + w] = left_bins_word(info, w, info.wide);
             t.split_gain[node] = static_cast<float>(info.gain + g.cfg.min_gain_to_split);
             t.threshold_bin[node] = info.threshold;
             t.default_left[node] = static_cast<uint8_t>(info.default_left);
@@ -3324,7 +3293,9 @@ __device__ void apply_commits(const GrowState &g, const AdvShared<MAXL> &s, uint
 // gain as f32 in .y; leaves not below a committed leaf (the committed tree's nodes) get -1. Pointer jumping over
 // parent links kept in the s.ckey words: a leaf's link is its parent until it meets a committed leaf, each round
 // takes the minimum with its link's and doubles the link's reach, so ceil(log2(depth)) + 1 rounds end it (at most
-// 16, which covers any tree of the sizes here). Block-wide.
+// 16, which covers any tree of the sizes here). Before the rounds, each leaf walks up to BOUND_WALK links by itself, which
+// ends most trees' without a round (a round is two barriers). Block-wide.
+constexpr int BOUND_WALK = 8;
 template <uint32_t MAXL>
 __device__ void frontier_bounds(AdvShared<MAXL> &s, uint32_t ntent, uint32_t n) {
     constexpr uint32_t PER = (AdvShared<MAXL>::TCAP + 511) / 512;  // leaves a thread (blocks of at least 512)
@@ -3350,10 +3321,29 @@ __device__ void frontier_bounds(AdvShared<MAXL> &s, uint32_t ntent, uint32_t n) 
     __syncthreads();
     for (uint32_t id = tid; id < n; id += nt) link[s.leaf_t[id]] = UNDER | NONE;  // the committed leaves: the path's top
     __syncthreads();
-    for (int round = 0; round < 16; ++round) {
+    for (int round = -1; round < 16; ++round) {
         uint32_t nl[PER];
         float nb[PER];
         bool moved = false;
+        if (round < 0) {
+#pragma unroll
+            for (uint32_t i = 0; i < PER; ++i) {
+                const uint32_t k = tid + nt * i;
+                nl[i] = NONE;
+                nb[i] = 0.0f;
+                if (k >= ntent) continue;
+                uint32_t l = link[k];
+                float b = bw[k].x;
+                for (int w = 0; w < BOUND_WALK && (l & NONE) != NONE; ++w) {
+                    const uint32_t u = l & NONE, lu = link[u];
+                    b = fminf(b, bw[u].y);  // .y: the leaf's own gain, which no round changes
+                    l = (l & UNDER) | lu;
+                }
+                nl[i] = l;
+                nb[i] = b;
+                moved = moved || (l & NONE) != NONE;
+            }
+        } else
 #pragma unroll
         for (uint32_t i = 0; i < PER; ++i) {
             const uint32_t k = tid + nt * i;
@@ -3451,17 +3441,20 @@ __device__ uint32_t pool_threshold(AdvShared<MAXL> &s, uint32_t ntent, uint32_t 
     return prefix;
 }
 
+// The control block's words that advance reads.
+struct AdvState {
+    uint32_t n0, ntent, pending0, slot0, epoch0, expansions0, steps0;
+};
+__device__ __forceinline__ AdvState adv_state(const GrowCtl *ctl) {
+    return AdvState{ctl->num_leaves, ctl->ntent, ctl->pending, ctl->next_slot, ctl->epoch, ctl->expansions, ctl->steps};
+}
+
+// advance's LDS copies of the first `ntk` speculative leaves' keys and of the committed leaves. Block-wide; the caller
+// synchronizes.
 template <uint32_t MAXL>
-__device__ void advance(const GrowState &g, StepPlan &next, void *scratch) {
-    AdvShared<MAXL> &s = *reinterpret_cast<AdvShared<MAXL> *>(scratch);
-    GrowCtl *ctl = g.ctl;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, nt = blockDim.x;
-    if (ctl->done) return;
-    const uint32_t n0 = ctl->num_leaves, ntent = ctl->ntent, L = g.num_leaves;
-    const uint32_t pending0 = ctl->pending, slot0 = ctl->next_slot, epoch0 = ctl->epoch;
-    const uint32_t expansions0 = ctl->expansions, steps0 = ctl->steps;
-    __syncthreads();  // every thread has read the control block before thread 0 updates it
-    for (uint32_t k = tid; k < ntent; k += nt) {
+__device__ __forceinline__ void advance_load(const GrowState &g, AdvShared<MAXL> &s, uint32_t n0, uint32_t ntk) {
+    const uint32_t tid = threadIdx.x, nt = blockDim.x;
+    for (uint32_t k = tid; k < ntk; k += nt) {
         const TKey key = g.tk[k];
         s.gain[k] = key.gain;
         s.meta[k] = key_meta(key);
@@ -3476,7 +3469,16 @@ __device__ void advance(const GrowState &g, StepPlan &next, void *scratch) {
         s.ncand = 0;
         s.nnan = 0;
     }
-    __syncthreads();
+}
+
+// With every key in LDS (advance_load), after a barrier.
+template <uint32_t MAXL>
+__device__ void advance(const GrowState &g, StepPlan &next, AdvShared<MAXL> &s, const AdvState &st) {
+    GrowCtl *ctl = g.ctl;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, nt = blockDim.x;
+    const uint32_t n0 = st.n0, ntent = st.ntent, L = g.num_leaves;
+    const uint32_t pending0 = st.pending0, slot0 = st.slot0, epoch0 = st.epoch0;
+    const uint32_t expansions0 = st.expansions0, steps0 = st.steps0;
     // the replay keys of the committed leaves for replay_lds and replay_reg (trees of more than 128 leaves), by the
     // whole block
     if (MAXL > LEAVES_SMALL || L > 128) {
@@ -3629,7 +3631,7 @@ __device__ void advance(const GrowState &g, StepPlan &next, void *scratch) {
             J.begin = l.begin;
             J.count = l.count;
             J.col = info.col;
-            J.wide = g.feats[info.feature].wide;
+            J.wide = info.wide;
 #pragma unroll
             for (uint32_t w = 0; w < 8; ++w) J.left_bins[w] = left_bins_word(info, w, J.wide);
             J.built_side = info.left_count <= info.right_count ? 0u : 1u;
@@ -3653,6 +3655,9 @@ __device__ void advance(const GrowState &g, StepPlan &next, void *scratch) {
             J.child_uh[0] = info.left_hess;
             J.child_ug[1] = info.right_grad;
             J.child_uh[1] = info.right_hess;
+            J.child_out[0] = info.left_output;
+            J.child_out[1] = info.right_output;
+            J.depth = l.depth + 1;
             J.kid = static_cast<int32_t>(ntent + 2 * lane);
         }
         // exclusive prefixes over lanes 0..njobs-1 (one wave)
@@ -3780,6 +3785,9 @@ template <uint32_t MAXL>
 __global__ __launch_bounds__(512) void k_root_select(GrowState g) {
     __shared__ SplitOut o;
     __shared__ __align__(16) uint8_t scratch[sizeof(AdvShared<MAXL>)];
+    AdvShared<MAXL> &s = *reinterpret_cast<AdvShared<MAXL> *>(scratch);
+    const AdvState st = adv_state(g.ctl);
+    const uint32_t done = g.ctl->done;
     ScanJob job = g.jobs[0];
     select_split(job, job.count, g.nf, g.cfg, grow_sg(g), grow_sh(g), &o, g.splittable);
     if (threadIdx.x == 0) {
@@ -3788,10 +3796,11 @@ __global__ __launch_bounds__(512) void k_root_select(GrowState g) {
         g.tk[0].gain = o.gain;
         g.tk[0].has = o.found ? 1u : 0u;
     }
-    __builtin_amdgcn_s_waitcnt(0);
+    if (done) return;
     __syncthreads();
-    __threadfence();
-    advance<MAXL>(g, g.plans[0], scratch);
+    advance_load(g, s, st.n0, st.ntent);
+    __syncthreads();
+    advance<MAXL>(g, g.plans[0], s, st);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -3807,9 +3816,8 @@ __global__ __launch_bounds__(512) void k_root_select(GrowState g) {
 //
 // Then, one launch each: k_step_children adds each job's partials, writes the built child's histogram, forms the sibling
 // by subtraction (learner.rs:356-371) and scans every (job, feature, child) of the byte slabs (k_step_reduce and
-// k_step_scan do so for two-byte slabs); k_step_select selects both children's splits of each job
-// (job_select), and its last block to finish runs advance. That hand-off is a counter the last arriving block
-// resets; no block ever waits for another.
+// k_step_scan do so for two-byte slabs); k_step_select, one block, selects both children's splits of every job and runs
+// advance.
 // ---------------------------------------------------------------------------------------------------------
 
 // A launch takes one slab, or (histogram only) several slabs of one kernel, k1 workgroups each: slab s of the
@@ -4631,7 +4639,6 @@ struct ScanStepArgs {
 };
 
 struct SelectArgs {
-    uint32_t *all_count;        // jobs selected; returned to 0 by the last one
     StepPlan *plan;             // this step's plan
     StepPlan *next;             // the next step's
 };
@@ -4642,119 +4649,6 @@ struct ReduceStepArgs {
     const ColGroup *cgs;        // [ncgw], the two-byte slabs'
     StepPlan *plan;
 };
-
-// The end of job j, by one block (learner.rs:294-352): both children's best splits (split.rs:866-880) from their
-// candidate slots' gains, a wave a child, while the other waves count the job's evaluated features; then their leaves in
-// the speculative tree and the job's leaf marked expanded (thread 0).
-__device__ void job_select(const GrowState &g, const JobPlan &J, uint32_t j) {
-    __shared__ SplitOut s_out[2];
-    __shared__ uint32_t s_used[16];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    GrowCtl *ctl = g.ctl;
-    const int64_t left = static_cast<int64_t>(J.left);
-    const int64_t right = J.parent_count - left;
-    if (!(left > 0 && right > 0)) {  // uniform over the block
-        if (threadIdx.x == 0) {
-            ctl->error = 1;
-            ctl->done = 1;
-            const uint32_t info[8] = {j, J.t, J.count, J.left, J.ntiles, J.groups, J.packed, 0u};
-            for (int k = 0; k < 8; ++k) ctl->err_info[k] = info[k];
-        }
-        return;
-    }
-    const int32_t kid = J.kid;
-    const int32_t depth = g.tl[J.t].depth + 1;
-    const int64_t min_pair = 2 * g.cfg.min_data_in_leaf;
-    const bool searched = J.hist && depth_allows(g, depth) && (left >= min_pair || right >= min_pair);
-    const uint32_t nw = blockDim.x >> 6;
-    // waves 0 and 1: the best split of the left and the right child; the others: the job's evaluated features
-    // (learner.rs:262-265), for the byte count
-    if (wave >= 2) {
-        const uint8_t *prow = g.splittable + static_cast<size_t>(J.t) * g.nf;
-        uint32_t used = 0;
-        for (uint32_t f0 = (wave - 2u) * 64u; f0 < g.nf; f0 += 64u * (nw - 2u)) {
-            const uint32_t f = f0 + lane;
-            used += static_cast<uint32_t>(__popcll(__ballot(f < g.nf && g.mask[f] != 0 && prow[f] != 0)));
-        }
-        if (lane == 0) s_used[wave] = used;
-    } else {
-        const uint32_t ch = wave;
-        SplitOut out = {};
-        if (searched) {
-            const size_t base = (static_cast<size_t>(j) * 2 + ch) * g.nslot;
-            double best = 0.0;
-            int bf = -1;
-            uint32_t bs = 0;
-            for (uint32_t s = lane; s < g.nslot; s += 64u) {
-                const double gv = g.cand_gain[base + s];
-                const int fv = g.cand_feat[base + s];
-                if (cand_better(gv, fv, best, bf)) {
-                    best = gv;
-                    bf = fv;
-                    bs = s;
-                }
-            }
-            int wf = bf;
-            wave_best(best, wf);
-            if (wf >= 0) {  // the winner, read where the scans left it (a feature is in one slot)
-                const uint32_t owner = static_cast<uint32_t>(__builtin_ctzll(__ballot(bf == wf)));
-                const uint32_t slot = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bs), owner));
-                const int64_t cnt = ch == 0 ? left : right;
-                out = split_out(g.cands[base + slot], wf, make_ctx(g.cfg, grow_sg(g), grow_sh(g), J.child_ug[ch], J.child_uh[ch], cnt), g.cfg);
-            }
-        }
-        if (lane == 0) s_out[ch] = out;
-    }
-    __syncthreads();
-    // the children's best splits, copied a dword a thread (no child-sized copy through one thread's stack)
-    static_assert(sizeof(SplitOut) % 4 == 0 && sizeof(SplitOut) / 4 <= 64, "a split copies in one wave");
-    if (threadIdx.x < 128) {
-        const uint32_t ch = threadIdx.x >> 6, d = threadIdx.x & 63u;
-        if (d < sizeof(SplitOut) / 4)
-            reinterpret_cast<uint32_t *>(&g.tl[kid + static_cast<int32_t>(ch)].best)[d] =
-                reinterpret_cast<const uint32_t *>(&s_out[ch])[d];
-    }
-    if (threadIdx.x == 0) {
-        const SplitOut &info = g.tl[J.t].best;
-        const uint32_t has[2] = {s_out[0].found ? 1u : 0u, s_out[1].found ? 1u : 0u};
-        const double gain[2] = {s_out[0].gain, s_out[1].gain};
-        const double lv = info.left_output, rv = info.right_output;
-        const double lh = info.left_hess, rh = info.right_hess;
-#pragma unroll
-        for (uint32_t ch = 0; ch < 2; ++ch) {
-            TLeaf &c = g.tl[kid + static_cast<int32_t>(ch)];
-            c.begin = ch == 0 ? J.begin : J.begin + J.left;
-            c.count = ch == 0 ? J.left : J.count - J.left;
-            c.ug = ch == 0 ? info.left_grad : info.right_grad;
-            c.uh = ch == 0 ? lh : rh;
-            c.cnt = ch == 0 ? left : right;
-            // the built child's histogram goes to the job's new slot, the other child keeps its parent's
-            c.slot = searched ? ((J.built_side == ch) ? J.built_slot : J.parent_slot) : -1;
-            c.has_best = searched ? has[ch] : 0u;
-            c.buf = 1u - J.src_buf;
-            c.rev = ch;  // the split step writes the left child first-first and the right child last-first
-            c.depth = depth;
-            c.state = T_LEAF;
-            c.kid = -1;
-            c.pad_ = 0;
-            const double v = ch == 0 ? lv : rv;
-            c.value = v != v ? 0.0 : v;
-            c.weight = (ch == 0 ? lh : rh) * grow_sh(g);
-            g.tk[kid + static_cast<int32_t>(ch)] = TKey{gain[ch], searched ? has[ch] : 0u, T_LEAF, -1, 0u};
-        }
-        g.tl[J.t].state = T_EXPANDED;
-        g.tk[J.t].state = T_EXPANDED;
-        if (J.hist) {  // the built child's histogram was made, searched or not
-            const double built_rows = J.built_side == 0 ? static_cast<double>(left) : static_cast<double>(right);
-            atomicAdd(&ctl->hist_rows, built_rows);
-            uint32_t used = 0;
-            for (uint32_t w = 2; w < nw; ++w) used += s_used[w];
-            atomicAdd(&ctl->hist_bins, built_rows * static_cast<double>(used));
-            atomicAdd(&ctl->hist_builds, 1.0);
-        }
-        atomicAdd(&ctl->part_rows, static_cast<double>(J.count));
-    }
-}
 
 // The children's histograms and candidates of each job over its byte slabs, one work item per (job, column group): the
 // built child's histogram of the group's four columns from the job's partials and its sibling's by subtraction in place
@@ -5160,26 +5054,157 @@ __global__ __launch_bounds__(256) void k_step_scan(GrowState g, ScanStepArgs a) 
     }
 }
 
-// Block j selects both children of job j (job_select); the last block to finish runs advance. grid: jcap blocks.
+// The end of a step, by one block: each job's children take their best splits (learner.rs:294-352, split.rs:866-880) and
+// become leaves of the speculative tree, then advance replays and plans the next step. What bounds it is the chain of
+// dependent loads of what other XCDs just wrote (about 1 us each), not its work: so one block does all jobs (a block a job
+// met through a counter, whose fences alone took several microseconds), loads everything whose address does not depend on
+// another load at once, keeps the new leaves' keys in LDS for the replay, and a plan carries what its children need of
+// their parent. 20.6 -> 15.4 us a step on 100k x 28, 37.4 -> 34.6 us on 10M x 128. One block, of 1024 threads for trees of
+// more than 512 leaves (up to 128 children a step: 76.5 us at 2047 leaves against 82.6 with 512 threads). MAXL: the
+// largest tree it takes.
+template <uint32_t MAXL> constexpr uint32_t select_threads() { return MAXL > LEAVES_SMALL ? 1024u : 512u; }
 template <uint32_t MAXL>
-__global__ __launch_bounds__(512) void k_step_select(GrowState g, SelectArgs a) {
+__global__ __launch_bounds__(select_threads<MAXL>()) void k_step_select(GrowState g, SelectArgs a) {
+    constexpr uint32_t NW = select_threads<MAXL>() / 64, BATCH = 4;
     __shared__ __align__(16) uint8_t scratch[sizeof(AdvShared<MAXL>)];
-    // the next plan stays empty unless advance writes it (it runs after every block has arrived, so after this):
-    // the steps after a finished tree do nothing without reading the control block
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    __shared__ int32_t s_feat[2 * JMAX];   // per (job, child), its best feature (-1: none) and that candidate's slot
+    __shared__ uint32_t s_slot[2 * JMAX];
+    __shared__ uint32_t s_bad;
+    AdvShared<MAXL> &s = *reinterpret_cast<AdvShared<MAXL> *>(scratch);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const StepPlan &P = *a.plan;
+    const AdvState st = adv_state(g.ctl);
+    const uint32_t done = g.ctl->done, njobs = P.njobs, pairs = 2u * njobs;
+    const uint32_t pj = tid < 2u * JMAX ? tid >> 1 : 0u, ch = tid & 1u;
+    const JobPlan &J = P.jobs[pj];  // thread p < pairs: child p % 2 of job p / 2
+    if (done || njobs == 0) {
+        // the next plan stays empty: the steps after a finished tree do nothing without reading the control block
+        if (tid == 0) {
+            a.next->njobs = 0;
+            a.next->total_groups = 0;
+            a.next->total_child = 0;
+            a.next->total_red = 0;
+            a.next->total_scan = 0;
+        }
+        return;
+    }
+    if (tid == 0) s_bad = 0;
+    // the keys of the leaves before this step's children; the children's are made below
+    advance_load(g, s, st.n0, st.ntent - pairs);
+    // each child's best candidate over its slots by (gain, lower feature), a wave BATCH children at a time
+    for (uint32_t p0 = wave; p0 < pairs; p0 += NW * BATCH) {
+        double gv[BATCH];
+        int fv[BATCH];
+#pragma unroll
+        for (uint32_t i = 0; i < BATCH; ++i) {
+            const uint32_t p = p0 + NW * i < pairs ? p0 + NW * i : p0;
+            const size_t at = static_cast<size_t>(p) * g.nslot + (lane < g.nslot ? lane : 0u);
+            gv[i] = g.cand_gain[at];
+            fv[i] = g.cand_feat[at];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < BATCH; ++i) {
+            const uint32_t p = p0 + NW * i;
+            if (p >= pairs) continue;  // uniform
+            double best = gv[i];
+            int bf = lane < g.nslot ? fv[i] : -1;
+            uint32_t bs = lane;
+            for (uint32_t x = lane + 64u; x < g.nslot; x += 64u) {
+                const double gx = g.cand_gain[static_cast<size_t>(p) * g.nslot + x];
+                const int fx = g.cand_feat[static_cast<size_t>(p) * g.nslot + x];
+                if (cand_better(gx, fx, best, bf)) {
+                    best = gx;
+                    bf = fx;
+                    bs = x;
+                }
+            }
+            int wf = bf;
+            wave_best(best, wf);
+            const unsigned long long at = __ballot(bf == wf);  // a feature is in one slot
+            if (wf >= 0 && lane == static_cast<uint32_t>(__builtin_ctzll(at))) s_slot[p] = bs;
+            if (lane == 0) s_feat[p] = wf;
+        }
+    }
+    if (g.count_work)  // the jobs' evaluated features (learner.rs:262-265), for the byte counts
+        for (uint32_t j = wave; j < njobs; j += NW) {
+            const JobPlan &Q = P.jobs[j];
+            const uint8_t *prow = g.splittable + static_cast<size_t>(Q.t) * g.nf;
+            uint32_t used = 0;
+            for (uint32_t f0 = 0; f0 < g.nf; f0 += 64u)
+                used += static_cast<uint32_t>(__popcll(__ballot(f0 + lane < g.nf && g.mask[f0 + lane] != 0 && prow[f0 + lane] != 0)));
+            if (lane == 0) {
+                if (Q.hist) {  // the built child's histogram was made, searched or not
+                    const double built = static_cast<double>(Q.built_side == 0 ? Q.left : Q.count - Q.left);
+                    atomicAdd(&g.ctl->hist_rows, built);
+                    atomicAdd(&g.ctl->hist_bins, built * static_cast<double>(used));
+                    atomicAdd(&g.ctl->hist_builds, 1.0);
+                }
+                atomicAdd(&g.ctl->part_rows, static_cast<double>(Q.count));
+            }
+        }
+    __syncthreads();
+    if (tid < pairs) {
+        const int64_t left = static_cast<int64_t>(J.left), right = J.parent_count - left;
+        if (!(left > 0 && right > 0)) {
+            if (ch == 0 && atomicExch(&s_bad, 1u) == 0u) {
+                const uint32_t info[8] = {pj, J.t, J.count, J.left, J.ntiles, J.groups, J.packed, 0u};
+                for (int k = 0; k < 8; ++k) g.ctl->err_info[k] = info[k];
+            }
+        } else {
+            const int64_t min_pair = 2 * g.cfg.min_data_in_leaf, cnt = ch == 0 ? left : right;
+            const bool searched = J.hist && depth_allows(g, J.depth) && (left >= min_pair || right >= min_pair);
+            const double ug = ch == 0 ? J.child_ug[0] : J.child_ug[1], uh = ch == 0 ? J.child_uh[0] : J.child_uh[1];
+            const uint32_t kid = static_cast<uint32_t>(J.kid) + ch;
+            TLeaf c;
+            c.best = SplitOut{};
+            const int bf = searched ? s_feat[tid] : -1;
+            if (bf >= 0)
+                c.best = split_out(g.cands[static_cast<size_t>(tid) * g.nslot + s_slot[tid]], bf,
+                                   make_ctx(g.cfg, grow_sg(g), grow_sh(g), ug, uh, cnt), g.cfg);
+            const uint32_t has = c.best.found ? 1u : 0u;
+            c.begin = ch == 0 ? J.begin : J.begin + J.left;
+            c.count = ch == 0 ? J.left : J.count - J.left;
+            c.ug = ug;
+            c.uh = uh;
+            c.cnt = cnt;
+            // the built child's histogram goes to the job's new slot, the other child keeps its parent's
+            c.slot = searched ? ((J.built_side == ch) ? J.built_slot : J.parent_slot) : -1;
+            c.has_best = has;
+            c.buf = 1u - J.src_buf;
+            c.rev = ch;  // the split step writes the left child first-first and the right child last-first
+            c.depth = J.depth;
+            c.state = T_LEAF;
+            c.kid = -1;
+            c.pad_ = 0;
+            const double v = ch == 0 ? J.child_out[0] : J.child_out[1];
+            c.value = v != v ? 0.0 : v;
+            c.weight = uh * grow_sh(g);
+            const TKey key{c.best.gain, has, T_LEAF, -1, 0u};
+            g.tl[kid] = c;
+            g.tk[kid] = key;
+            s.gain[kid] = key.gain;
+            s.meta[kid] = key_meta(key);
+            if (ch == 0) {  // the job's leaf, which has a split and is expanded now
+                g.tl[J.t].state = T_EXPANDED;
+                g.tk[J.t].state = T_EXPANDED;
+                s.meta[J.t] = key_meta(TKey{0.0, 1u, T_EXPANDED, J.kid, 0u});
+            }
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {  // empty unless advance writes it
         a.next->njobs = 0;
         a.next->total_groups = 0;
         a.next->total_child = 0;
         a.next->total_red = 0;
         a.next->total_scan = 0;
+        if (s_bad) {
+            g.ctl->error = 1;
+            g.ctl->done = 1;
+        }
     }
-    if (g.ctl->done) return;
-    StepPlan &P = *a.plan;
-    const uint32_t j = blockIdx.x;
-    if (j >= P.njobs) return;
-    job_select(g, P.jobs[j], j);
-    if (!arrive_last(a.all_count, P.njobs)) return;
-    advance<MAXL>(g, *a.next, scratch);
+    if (s_bad) return;  // uniform
+    advance<MAXL>(g, *a.next, s, st);
 }
 
 }  // namespace srocm
