@@ -88,7 +88,7 @@ def step_kernels(layout, quant_bins):
     (units of at most 7 and 15, i.e. num_grad_quant_bins up to 14, and no separate counters)."""
     out = {}
     for sl in layout:
-        dp = (4 if sl["row_bytes"] <= 1024 else 8) if sl["dense"] else 0
+        dp = next(d for d in (1, 2, 4, 8) if sl["row_bytes"] <= 256 * d) if sl["dense"] else 0
         codes = not sl["q32"] and quant_bins <= 14
         k = (f"k_step_rows<{sl['width']}, {'true' if sl['wide'] else 'false'}, {max(sl['pack'], 1)}, "
              f"{'true' if sl['q32'] else 'false'}, {dp}, {'true' if codes else 'false'}>")

@@ -940,7 +940,7 @@ struct Context {
                 Slab &s = out[si];
                 s.width = 128;
                 s.dense_row = 128 * per;
-                s.dense_passes = per <= 8 ? 4 : 8;  // 32 * per dwords a row, 64 a pass
+                s.dense_passes = per <= 2 ? 1 : (per <= 4 ? 2 : (per <= 8 ? 4 : 8));  // 32 * per dwords a row, 64 a pass
                 s.pos_word.resize(256ull * s.dense_passes);
                 for (uint32_t p = 0; p < s.pos_word.size(); ++p) s.pos_word[p] = 256u * 128u + p % 128;  // the spare row
                 s.slot_flat.assign(256ull * 128, 0u);
@@ -1419,6 +1419,8 @@ struct Context {
             case 34: k_hist<32, false, 2><<<grid, 1024, 0, stream>>>(a); break;
             case 66: k_hist<64, false, 2><<<grid, 1024, 0, stream>>>(a); break;
             case 130: k_hist<128, false, 2><<<grid, 1024, 0, stream>>>(a); break;
+            case 3001: k_hist<128, false, 1, false, 1><<<grid, 1024, 0, stream>>>(a); break;
+            case 3002: k_hist<128, false, 1, false, 2><<<grid, 1024, 0, stream>>>(a); break;
             case 3004: k_hist<128, false, 1, false, 4><<<grid, 1024, 0, stream>>>(a); break;
             case 3008: k_hist<128, false, 1, false, 8><<<grid, 1024, 0, stream>>>(a); break;
             case 1032: k_hist<32, false, 1, true><<<grid, 1024, 0, stream>>>(a); break;
@@ -2409,6 +2411,8 @@ void Context::grow(const srocm_grow_spec &spec, HostTree &tree, std::vector<sroc
                     SROCM_STEP_CASE(34, 32, false, 2, 0)
                     SROCM_STEP_CASE(66, 64, false, 2, 0)
                     SROCM_STEP_CASE(130, 128, false, 2, 0)
+                    SROCM_STEP_CASE(3001, 128, false, 1, 1)
+                    SROCM_STEP_CASE(3002, 128, false, 1, 2)
                     SROCM_STEP_CASE(3004, 128, false, 1, 4)
                     SROCM_STEP_CASE(3008, 128, false, 1, 8)
 #undef SROCM_STEP_CASE

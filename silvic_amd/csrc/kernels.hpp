@@ -419,33 +419,45 @@ __device__ __forceinline__ void dense_lanes(const uint32_t *pos_word, uint32_t l
 }
 
 // The rows list[c0 .. c1) of a dense slab into the LDS, UNROLL rows a wave at a time over NW waves (`wave` among
-// them); dwords past the row (dw_row) read as 0, i.e. bin 0 of spare positions.
-template <int W, int DP, int UNROLL, int NW = 16, bool CODES = false>
+// them); dwords past the row (dw_row) read as 0, i.e. bin 0 of spare positions. 16 dwords a lane are in flight whatever the
+// row's length (UNROLL = 16 / DP): what bounds it is the latency of the rows' gathers. A step's row ids and gradients are
+// one load each (lane u: row u, read across lanes as scalars), the ids a step ahead. With 4 passes for every row of up to
+// 1024 bytes, a 256-byte row took three passes of spare adds: 1M x 136 in 256-byte rows, root k_hist 172 -> 71 us,
+// k_step_rows 72.3 -> 29.1 us a launch.
+template <int DP> constexpr int dense_unroll() { return 16 / DP; }
+template <int W, int DP, int NW = 16, bool CODES = false>
 __device__ __forceinline__ void hist_list_dense(int32_t *lds, const uint32_t *list, uint32_t c0, uint32_t c1,
                                                 const int32_t *gh, const uint32_t *bins32, uint32_t dw_row,
                                                 const uint32_t (&xs)[4], const uint32_t (&cols)[DP][4],
                                                 uint32_t wave = threadIdx.x >> 6, const uint8_t *codes = nullptr) {
+    constexpr int UNROLL = dense_unroll<DP>();
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t last = c1 - 1;
-    for (uint32_t base = c0 + wave * UNROLL; base < c1; base += NW * UNROLL) {
+    uint32_t base = c0 + __builtin_amdgcn_readfirstlane(wave) * UNROLL;
+    if (base >= c1) return;
+    const uint32_t last = c1 - 1, mine = lane < UNROLL ? lane : UNROLL - 1;
+    uint32_t cidx = list[min(base + mine, last)];
+    for (; base < c1; base += NW * UNROLL) {
+        int32_t gl;
+        if constexpr (CODES) gl = code_word(codes[min(base + mine, last)]);
+        else gl = gh[cidx];
         uint32_t r[UNROLL];
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) r[u] = list[min(base + u, last)];
-        int32_t gq[UNROLL];
+        for (int u = 0; u < UNROLL; ++u) r[u] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(cidx), u));
+        cidx = list[min(base + NW * UNROLL + mine, last)];
         uint32_t dw[UNROLL][DP];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
-            if constexpr (CODES) gq[u] = code_word(codes[min(base + u, last)]);
-            else gq[u] = gh[r[u]];
+            const uint32_t *row = bins32 + static_cast<size_t>(r[u]) * dw_row;
 #pragma unroll
             for (int p = 0; p < DP; ++p) {
                 const uint32_t d = 64u * p + lane;
-                dw[u][p] = d < dw_row ? bins32[static_cast<size_t>(r[u]) * dw_row + d] : 0u;
+                dw[u][p] = d < dw_row ? row[d] : 0u;
             }
         }
+        if (base + mine >= c1) gl = 0;
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
-            const int32_t gv = base + u < c1 ? gq[u] : 0;
+            const int32_t gv = __builtin_amdgcn_readlane(gl, u);
 #pragma unroll
             for (int p = 0; p < DP; ++p) add_row_bins<W>(lds, dw[u][p], gv, 0, xs, cols[p]);
         }
@@ -498,7 +510,7 @@ __global__ __launch_bounds__(1024) void k_hist(HistArgs a) {
     for (uint32_t chunk = start; chunk < end; chunk += a.flush_rows) {
         uint32_t cend = end - chunk > a.flush_rows ? chunk + a.flush_rows : end;
         if constexpr (DP > 0) {
-            hist_list_dense<W, DP, DP <= 4 ? 4 : 2>(lds, rows, chunk, cend, a.gh, bins32, a.dw_row, xs, dcols);
+            hist_list_dense<W, DP>(lds, rows, chunk, cend, a.gh, bins32, a.dw_row, xs, dcols);
         } else {
             uint32_t last = cend - 1;
             uint32_t base = chunk + wave * RPW * UNROLL;
@@ -4233,7 +4245,7 @@ __device__ __forceinline__ void step_hist(int32_t *lds, const uint32_t *list, ui
                                           const uint32_t (&dcols)[DP ? DP : 1][4], uint32_t wave = threadIdx.x >> 6,
                                           const uint8_t *codes = nullptr) {
     if constexpr (DP > 0)
-        hist_list_dense<W, DP, DP <= 4 ? 2 : 1, NW, CODES>(lds, list, c0, c1, gh, bins32, dw_row, xs, dcols, wave, codes);
+        hist_list_dense<W, DP, NW, CODES>(lds, list, c0, c1, gh, bins32, dw_row, xs, dcols, wave, codes);
     else if constexpr (W == 128 && !WIDE && PACK == 1 && !Q32)
         hist_list_pairs<UNROLL * 3 / 4, NW, CODES>(lds, list, c0, c1, gh, bins32, wave, codes);
     else hist_list<W, WIDE, PACK, Q32, UNROLL, NW, CODES>(lds, list, c0, c1, gh, bins32, wave, codes);

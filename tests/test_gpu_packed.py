@@ -178,3 +178,25 @@ def test_dense_boosting_matches_the_oracle():
         compare_trees(d, ot, f"tree {i}", exact_values=False)
     assert np.array_equal(t.backend.scores(0), o.scores)
     t.backend.close()
+
+
+# A dense slab's rows are read in 1, 2, 4 or 8 passes of 256 bytes: rows of exactly one, two and four passes, row counts that
+# end inside a wave's rows, with carried gradient codes (4 bins) and with gathered words (16).
+@pytest.mark.parametrize("full,few,per", [(136, 0, 2), (5, 470, 4), (0, 1000, 8)])
+@pytest.mark.parametrize("qbins", [4, 16])
+def test_dense_rows_of_every_pass_count_match_the_oracle(rocm, full, few, per, qbins):
+    say("dense passes", full, few, qbins)
+    rows = 50_013
+    parts = [silvic_amd.synthetic(c, rows=rows, cols=n, seed=per) for c, n in ((2, full), (4, few)) if n]
+    data = parts[0] if len(parts) == 1 else joined(*parts)
+    g, h = binary_gradients(data, per)
+    p = oracle.default_params(num_leaves=31, num_grad_quant_bins=qbins)
+    o_tree, _, o_part = oracle.grow_tree(data, g, h, p, renew=False)
+    spec, packed = quantized_setup(rocm, data, g, h, seed=p.data_random_seed, num_bins=qbins)
+    check_layout(rocm, dict(dense=1, per=per))
+    n = rocm.reset_partition()
+    assert np.array_equal(rocm.histogram((7, n - 20)), oracle.histogram(data, packed, qbins, np.arange(7, n - 13, dtype=np.uint32)))
+    mask = oracle.feature_mask(data.features, 1.0, 2, 0)
+    d = rocm.grow(p.cfg, p.num_leaves, p.max_depth, spec.grad_scale, spec.hess_scale, mask, (0, n), n)
+    compare_trees(d, dict(o_tree), f"dense passes {per}")
+    assert np.array_equal(rocm.partition_rows(n), o_part[:n])
