@@ -7,6 +7,7 @@ total_bins`` float64 integers in quantized mode.
 """
 
 import ctypes as C
+import struct
 
 import numpy as np
 
@@ -19,6 +20,14 @@ DEFAULT_LABEL_GAIN = [float((1 << i) - 1) for i in range(31)]
 
 def _p(a, t):
     return a.ctypes.data_as(C.POINTER(t))
+
+
+def _feature_table(features):
+    """The ``srocm_feature`` array of ``features``, packed in one call (a ctypes constructor a feature took longer than the
+    search it describes)."""
+    flat = [v for f in features for v in (f.num_bins, f.group, f.column, f.hist_offset, f.kind, bool(f.nan_bin))]
+    n = max(1, len(features))
+    return (_abi.Feature * n).from_buffer_copy(struct.pack(f"={6 * n}I", *(flat or [0] * 6)))
 
 
 class RocmBackend:
@@ -207,9 +216,7 @@ class RocmBackend:
 
     def find_best_split_slot(self, slot, features, evaluate, sums, grad_scale, hess_scale, cfg):
         ev = np.ascontiguousarray(evaluate, dtype=np.uint8)
-        feats = (_abi.Feature * max(1, len(features)))()
-        for i, f in enumerate(features):
-            feats[i] = _abi.Feature(f.num_bins, f.group, f.column, f.hist_offset, f.kind, int(bool(f.nan_bin)))
+        feats = _feature_table(features)
         out = _abi.SplitInfo()
         spl = np.zeros(len(features), np.uint8)
         s = _abi.Sums(*sums)
@@ -222,9 +229,7 @@ class RocmBackend:
         """``split::find_best_split`` (split.rs:919-961) on the device: returns (SplitInfo, splittable bools)."""
         hist = np.ascontiguousarray(hist, dtype=np.float64)
         ev = np.ascontiguousarray(evaluate, dtype=np.uint8)
-        feats = (_abi.Feature * max(1, len(features)))()
-        for i, f in enumerate(features):
-            feats[i] = _abi.Feature(f.num_bins, f.group, f.column, f.hist_offset, f.kind, int(bool(f.nan_bin)))
+        feats = _feature_table(features)
         out = _abi.SplitInfo()
         spl = np.zeros(len(features), np.uint8)
         s = _abi.Sums(*sums)

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -411,7 +412,7 @@ struct Context {
     int64_t max_gq = 1, max_hq = 1;  // the last quantization's largest |g| and h units
     bool quantized_once = false;
 
-    Pinned<int64_t> h_hist;
+    Pinned<double> h_hist;  // a histogram on its way to the host (k_hist_to_host), or a host histogram for the device
     Pinned<uint32_t> h_u32;
     Pinned<uint8_t> h_result;
     Pinned<uint8_t> h_stage;  // per-split uploads (jobs, evaluate flags), rewritten only after a sync
@@ -475,6 +476,7 @@ struct Context {
             (void)hipEventDestroy(e.second);
         }
         for (auto e : prof.pool) (void)hipEventDestroy(e);
+        for (auto e : back_events) (void)hipEventDestroy(e);
         if (copy_stream) (void)hipStreamDestroy(copy_stream);
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -1348,7 +1350,6 @@ struct Context {
         a.row_offset = row_offset;
         a.fraction = bag.fraction;
         run_partition(a, static_cast<uint32_t>(rows));
-        hip_check(hipMemcpyAsync(h_u32.p, scalars.p, 4, hipMemcpyDeviceToHost, stream), "read bag count");
         sync();
         part_len = h_u32.p[0];
         return part_len;
@@ -1465,8 +1466,13 @@ struct Context {
 
     DevBuf<int64_t> tmp_hist;
 
-    void histogram_to_host(double *out) {
-        hip_check(hipMemcpyAsync(h_hist.p, tmp_hist.p, 2 * total_bins * sizeof(int64_t), hipMemcpyDeviceToHost, stream), "read histogram");
+    // A device histogram into the host's buffer: converted on the device into pinned memory, the stream waited for, copied.
+    void histogram_to_host(const int64_t *d, double *out) {
+        h_hist.alloc(2 * total_bins);
+        k_hist_to_host<<<std::min<uint32_t>(div_up(std::max<uint64_t>(total_bins, 1), 256), cus), 256, 0, stream>>>(d, h_hist.p, total_bins, nullptr, nullptr);
+        launch_check("k_hist_to_host");
+        sync();
+        std::memcpy(out, h_hist.p, 2 * total_bins * sizeof(double));
     }
 
     void histogram(srocm_leaf_range leaf, int quantized, double *out, size_t len) {
@@ -1477,15 +1483,12 @@ struct Context {
         if (len != 2 * total_bins) fail(SROCM_ERR_DEVICE, "histogram buffer of " + std::to_string(len) + " values, expected " + std::to_string(2 * total_bins));
         if (!quantized_once) fail(SROCM_ERR_DEVICE, "histogram before quantize");
         tmp_hist.alloc(2 * total_bins);
-        h_hist.alloc(2 * total_bins);
         if (leaf.count == 0) {
             std::fill(out, out + len, 0.0);
             return;
         }
         launch_hist(leaf.begin, leaf.count, nullptr, 0, tmp_hist.p, nullptr, used_columns());
-        histogram_to_host(out);
-        sync();
-        for (size_t i = 0; i < len; ++i) out[i] = static_cast<double>(h_hist.p[i]);
+        histogram_to_host(tmp_hist.p, out);
     }
 
     // histogram() into a caller-owned device buffer (i64 {g, h} per bin), with the partials in the scratch array:
@@ -1527,6 +1530,7 @@ struct Context {
         a.dst = part2.p;
         a.block_left = block_left.p;
         a.dev_left = scalars.p;
+        a.host_left = h_u32.p;
         a.begin = begin;
         a.count = count;
         return a;
@@ -1564,7 +1568,8 @@ struct Context {
             fail(SROCM_ERR_DEVICE, "split on a column without a feature");
         int32_t nt = group_col_nt[split.group][split.column];
         if (leaf.count == 0) {
-            hip_check(hipMemsetAsync(scalars.p, 0, 4, stream), "zero left");
+            sync();  // no launch of an earlier call still writes it
+            h_u32.p[0] = 0;
             return;
         }
         PartArgs a = part_args(leaf.begin, leaf.count);
@@ -1580,7 +1585,6 @@ struct Context {
         check_range(leaf);
         ensure_order();
         enqueue_partition(leaf, split);
-        hip_check(hipMemcpyAsync(h_u32.p, scalars.p, 4, hipMemcpyDeviceToHost, stream), "read left count");
         sync();
         return h_u32.p[0];
     }
@@ -1594,14 +1598,10 @@ struct Context {
         if (len != 2 * total_bins) fail(SROCM_ERR_DEVICE, "histogram buffer of " + std::to_string(len) + " values, expected " + std::to_string(2 * total_bins));
         if (side > 1) fail(SROCM_ERR_DEVICE, "bad side");
         tmp_hist.alloc(2 * total_bins);
-        h_hist.alloc(2 * total_bins);
         enqueue_partition(leaf, split);
         if (leaf.count) launch_hist(leaf.begin, leaf.count, scalars.p, side, tmp_hist.p, nullptr, used_columns());
         else hip_check(hipMemsetAsync(tmp_hist.p, 0, 2 * total_bins * 8, stream), "zero histogram");
-        histogram_to_host(out);
-        hip_check(hipMemcpyAsync(h_u32.p, scalars.p, 4, hipMemcpyDeviceToHost, stream), "read left count");
-        sync();
-        for (size_t i = 0; i < len; ++i) out[i] = static_cast<double>(h_hist.p[i]);
+        histogram_to_host(tmp_hist.p, out);
         return h_u32.p[0];
     }
 
@@ -1769,7 +1769,55 @@ struct Context {
         require_loaded();
         DevData &d = dataset(i);
         if (len != d.rows) fail(SROCM_ERR_DEVICE, "scores buffer of " + std::to_string(len) + " values, expected " + std::to_string(d.rows));
-        if (len) hip_check(hipMemcpyAsync(out, d.scores.p, len * 4, hipMemcpyDeviceToHost, stream), "read scores");
+        copy_out(out, d.scores.p, len * 4);
+    }
+
+    // Device memory into the caller's (pageable) memory, after what is queued on the stream: in pieces through pinned
+    // staging, a few host threads copying each piece out as it lands (the runtime's own pageable copy, one thread through
+    // its staging, moved 12 MB of scores in 800 us). The staging (STAGE_BYTES at most) and the threads are kept.
+    static constexpr size_t STAGE_PIECE = size_t(1) << 20, STAGE_PIECES = 16;
+    Pinned<uint8_t> h_back;
+    std::vector<hipEvent_t> back_events;
+    std::unique_ptr<srocm_rank::WorkPool> copy_pool;
+    void copy_out(void *dst, const void *src, size_t bytes) {
+        if (bytes <= STAGE_PIECE) {  // one piece: no threads
+            if (bytes) {
+                h_back.alloc(bytes);
+                hip_check(hipMemcpyAsync(h_back.p, src, bytes, hipMemcpyDeviceToHost, stream), "read back");
+            }
+            sync();
+            if (bytes) std::memcpy(dst, h_back.p, bytes);
+            return;
+        }
+        h_back.alloc(STAGE_PIECE * STAGE_PIECES);
+        while (back_events.size() < STAGE_PIECES) {
+            hipEvent_t e = nullptr;
+            hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+            back_events.push_back(e);
+        }
+        if (!copy_pool) copy_pool = std::make_unique<srocm_rank::WorkPool>(4);
+        for (size_t at = 0; at < bytes; at += STAGE_PIECE * STAGE_PIECES) {
+            const size_t part = std::min(bytes - at, STAGE_PIECE * STAGE_PIECES), pieces = (part + STAGE_PIECE - 1) / STAGE_PIECE;
+            for (size_t k = 0; k < pieces; ++k) {
+                const size_t o = k * STAGE_PIECE, n = std::min(STAGE_PIECE, part - o);
+                hip_check(hipMemcpyAsync(h_back.p + o, static_cast<const uint8_t *>(src) + at + o, n, hipMemcpyDeviceToHost, stream), "read back");
+                hip_check(hipEventRecord(back_events[k], stream), "event");
+            }
+            std::atomic<int> err{0};
+            const std::function<void(unsigned)> work = [&](unsigned w) {
+                for (size_t k = w; k < pieces; k += copy_pool->size()) {
+                    const hipError_t e = hipEventSynchronize(back_events[k]);
+                    if (e != hipSuccess) {
+                        err.store(static_cast<int>(e));
+                        return;
+                    }
+                    const size_t o = k * STAGE_PIECE;
+                    std::memcpy(static_cast<uint8_t *>(dst) + at + o, h_back.p + o, std::min(STAGE_PIECE, part - o));
+                }
+            };
+            copy_pool->run(work);
+            hip_check(static_cast<hipError_t>(err.load()), "read back");
+        }
         sync();
     }
 
@@ -1820,7 +1868,6 @@ struct Context {
         enqueue_partition(leaf, split);
         if (leaf.count) launch_hist(leaf.begin, leaf.count, scalars.p, side, d, nullptr, used_columns());
         else hip_check(hipMemsetAsync(d, 0, 2 * total_bins * 8, stream), "zero histogram");
-        hip_check(hipMemcpyAsync(h_u32.p, scalars.p, 4, hipMemcpyDeviceToHost, stream), "read left count");
         sync();
         return h_u32.p[0];
     }
@@ -1838,37 +1885,47 @@ struct Context {
     void read_slot(uint32_t slot, double *out, size_t len) {
         require_loaded();
         if (len != 2 * total_bins) fail(SROCM_ERR_DEVICE, "histogram buffer of " + std::to_string(len) + " values, expected " + std::to_string(2 * total_bins));
-        const int64_t *d = slot_ptr(slot);
-        h_hist.alloc(2 * total_bins);
-        hip_check(hipMemcpyAsync(h_hist.p, d, 2 * total_bins * 8, hipMemcpyDeviceToHost, stream), "read histogram slot");
-        sync();
-        for (size_t i = 0; i < len; ++i) out[i] = static_cast<double>(h_hist.p[i]);
+        histogram_to_host(slot_ptr(slot), out);
     }
 
     void find_best_split_slot(uint32_t slot, const srocm_feature *features, uint32_t num_features, const uint8_t *evaluate,
                               const srocm_sums &sums, double sg, double sh, const srocm_split_config &cfg,
                               srocm_split_info *out, uint8_t *splittable) {
         require_loaded();
-        find_best_split_dev(slot_ptr(slot), 2 * total_bins, features, num_features, evaluate, sums, sg, sh, cfg, out, splittable);
+        find_best_split_on<int64_t>(slot_ptr(slot), 2 * total_bins, features, num_features, evaluate, sums, sg, sh, cfg, out, splittable);
     }
 
     // split.rs:919-961 on a host histogram over an explicit feature table (no loaded dataset needed)
     void find_best_split(const double *hist, size_t len, const srocm_feature *features, uint32_t num_features,
                          const uint8_t *evaluate, const srocm_sums &sums, double sg, double sh,
                          const srocm_split_config &cfg, srocm_split_info *out, uint8_t *splittable) {
-        std::vector<int64_t> units(len);
-        for (size_t i = 0; i < len; ++i) units[i] = static_cast<int64_t>(hist[i]);
-        DevBuf<int64_t> dh;
-        dh.alloc(std::max<size_t>(len, 1));
-        if (len) hip_check(hipMemcpyAsync(dh.p, units.data(), len * 8, hipMemcpyHostToDevice, stream), "upload histogram");
-        find_best_split_dev(dh.p, len, features, num_features, evaluate, sums, sg, sh, cfg, out, splittable);
+        h_hist.alloc(std::max<size_t>(len, 1));
+        if (len) std::memcpy(h_hist.p, hist, len * sizeof(double));
+        find_best_split_on<double>(h_hist.p, len, features, num_features, evaluate, sums, sg, sh, cfg, out, splittable);
     }
 
-    // find_best_split over `len` int64 units on the device (an uploaded host histogram, or a histogram slot)
-    void find_best_split_dev(const int64_t *dh, size_t len, const srocm_feature *features, uint32_t num_features,
-                             const uint8_t *evaluate, const srocm_sums &sums, double sg, double sh,
-                             const srocm_split_config &cfg, srocm_split_info *out, uint8_t *splittable) {
+    // The split search's workspaces, kept from one call to the next: the feature table as the device last got it (uploaded
+    // again when its contents differ), the candidates, the categorical orders, and pinned memory that the kernels read the
+    // evaluated flags from and write the result to. (Allocating and freeing them in each call, nine copies and two waits
+    // took most of a call's 170 us.)
+    struct SplitResult {
+        SplitOut split;
+        uint8_t order[256];
+    };
+    std::vector<FeatDev> split_feats_host;
+    DevBuf<FeatDev> split_feats;
+    DevBuf<FeatCand> split_cands;
+    DevBuf<uint8_t> split_order;
+    Pinned<SplitResult> h_split;
+    Pinned<uint8_t> h_split_flags;  // evaluated, then splittable
+
+    // find_best_split over `len` units of type T where the device reads them: a histogram slot, or pinned host memory
+    template <class T>
+    void find_best_split_on(const T *hist, size_t len, const srocm_feature *features, uint32_t num_features,
+                            const uint8_t *evaluate, const srocm_sums &sums, double sg, double sh,
+                            const srocm_split_config &cfg, srocm_split_info *out, uint8_t *splittable) {
         std::vector<FeatDev> fd(num_features);
+        bool narrow = false, wide = false, cats = false;
         for (uint32_t f = 0; f < num_features; ++f) {
             const srocm_feature &m = features[f];
             if (m.num_bins > 1024 || (m.num_bins > 256 && m.kind != SROCM_BINS_NUMERICAL))
@@ -1876,80 +1933,35 @@ struct Context {
             if (m.num_bins && static_cast<uint64_t>(m.hist_offset) + m.num_bins > len / 2)
                 fail(SROCM_ERR_DEVICE, "feature " + std::to_string(f) + " lies outside the histogram");
             fd[f] = FeatDev{m.num_bins, m.hist_offset, m.kind, m.nan_bin, 0u, m.num_bins > 256 ? 1u : 0u};
+            (fd[f].wide ? wide : narrow) = true;
+            cats = cats || m.kind == SROCM_BINS_CATEGORICAL;
         }
-        DevBuf<FeatDev> dfd;
-        DevBuf<ScanJob> dj;
-        DevBuf<FeatCand> dc;
-        DevBuf<SplitOut> dso;
-        DevBuf<uint8_t> dsp, dev, dorder;
-        dorder.alloc(static_cast<size_t>(std::max<uint32_t>(num_features, 1)) * 256);
-        dfd.alloc(std::max<uint32_t>(num_features, 1));
-        dj.alloc(1);
-        dc.alloc(std::max<uint32_t>(num_features, 1));
-        dso.alloc(1);
-        dsp.alloc(std::max<uint32_t>(num_features, 1));
-        dev.alloc(std::max<uint32_t>(num_features, 1));
-        if (num_features) {
-            hip_check(hipMemcpyAsync(dfd.p, fd.data(), num_features * sizeof(FeatDev), hipMemcpyHostToDevice, stream), "upload features");
-            hip_check(hipMemcpyAsync(dev.p, evaluate, num_features, hipMemcpyHostToDevice, stream), "upload evaluate");
+        const size_t n = std::max<uint32_t>(num_features, 1);
+        split_cands.alloc(n);
+        h_split.alloc(1);
+        h_split_flags.alloc(2 * n);
+        if (cats) split_order.alloc(n * 256);
+        if (fd.size() != split_feats_host.size() || (num_features && std::memcmp(fd.data(), split_feats_host.data(), num_features * sizeof(FeatDev)) != 0)) {
+            split_feats_host.clear();  // unknown until the upload is queued
+            split_feats.alloc(n);
+            if (num_features) hip_check(hipMemcpy(split_feats.p, fd.data(), num_features * sizeof(FeatDev), hipMemcpyHostToDevice), "upload features");
+            split_feats_host = fd;
         }
-        ScanJob job{dh, sums.grad, sums.hess, sums.count, dc.p};
-        hip_check(hipMemcpyAsync(dj.p, &job, sizeof(job), hipMemcpyHostToDevice, stream), "upload job");
-        if (num_features) {
-            // numerical byte features of 2..64 bins go in scan units of several (k_split_scan_seg), as in a tree
-            std::vector<uint8_t> seg(num_features, 0);
-            std::vector<int32_t> ufeat;
-            std::vector<uint32_t> usegl;
-            for (uint32_t segl : {4u, 16u}) {
-                std::vector<int32_t> members;
-                for (uint32_t f = 0; f < num_features; ++f) {
-                    const FeatDev &x = fd[f];
-                    if (x.kind == SROCM_BINS_NUMERICAL && !x.wide && x.num_bins >= 2 && x.num_bins <= 64 &&
-                        (x.num_bins > 16 ? 16u : 4u) == segl) {
-                        members.push_back(static_cast<int32_t>(f));
-                        seg[f] = 1;
-                    }
-                }
-                const size_t per = 64 / segl;
-                for (size_t b = 0; b < members.size(); b += per) {
-                    for (size_t k = 0; k < UNIT_FEATS; ++k) ufeat.push_back(k < per && b + k < members.size() ? members[b + k] : -1);
-                    usegl.push_back(segl);
-                }
-            }
-            DevBuf<uint8_t> dseg;
-            DevBuf<int32_t> dufeat;
-            DevBuf<uint32_t> dusegl;
-            dseg.alloc(num_features);
-            hip_check(hipMemcpyAsync(dseg.p, seg.data(), num_features, hipMemcpyHostToDevice, stream), "upload scan units");
-            dim3 grid(div_up(num_features, 4), 1);
-            bool narrow = false, wide = false;
-            for (const FeatDev &x : fd) (x.wide ? wide : narrow) = true;
-            if (narrow) k_split_scan<false><<<grid, 256, 0, stream>>>(dj.p, dfd.p, dev.p, num_features, cfg_dev(cfg), sg, sh, dorder.p, nullptr, dseg.p);
-            if (wide) k_split_scan<true><<<grid, 256, 0, stream>>>(dj.p, dfd.p, dev.p, num_features, cfg_dev(cfg), sg, sh, dorder.p, nullptr);
-            launch_check("k_split_scan");
-            if (!usegl.empty()) {
-                dufeat.alloc(ufeat.size());
-                dusegl.alloc(usegl.size());
-                hip_check(hipMemcpyAsync(dufeat.p, ufeat.data(), ufeat.size() * 4, hipMemcpyHostToDevice, stream), "upload scan units");
-                hip_check(hipMemcpyAsync(dusegl.p, usegl.data(), usegl.size() * 4, hipMemcpyHostToDevice, stream), "upload scan units");
-                k_split_scan_seg<<<dim3(div_up(usegl.size(), 4), 1), 256, 0, stream>>>(dj.p, dfd.p, dev.p, dufeat.p, dusegl.p,
-                                                                                      static_cast<uint32_t>(usegl.size()), cfg_dev(cfg), sg, sh);
-                launch_check("k_split_scan_seg");
-            }
-            sync();  // the unit buffers are locals
-        }
-        k_split_select<<<1, 256, 0, stream>>>(dj.p, num_features, cfg_dev(cfg), sg, sh, dso.p, dsp.p);
+        if (num_features) std::memcpy(h_split_flags.p, evaluate, num_features);
+        const ScanJob job{reinterpret_cast<const int64_t *>(hist), sums.grad, sums.hess, sums.count, split_cands.p};
+        uint8_t *order = cats ? split_order.p : nullptr;
+        const uint32_t grid = div_up(num_features, 4);
+        if (narrow) k_split_scan<false, T><<<grid, 256, 0, stream>>>(job, nullptr, split_feats.p, h_split_flags.p, num_features, cfg_dev(cfg), sg, sh, order, nullptr);
+        if (wide) k_split_scan<true, T><<<grid, 256, 0, stream>>>(job, nullptr, split_feats.p, h_split_flags.p, num_features, cfg_dev(cfg), sg, sh, order, nullptr);
+        launch_check("k_split_scan");
+        k_split_select<<<1, 256, 0, stream>>>(job, num_features, cfg_dev(cfg), sg, sh, order, &h_split.p->split, h_split.p->order, h_split_flags.p + n);
         launch_check("k_split_select");
-        SplitOut o;
-        hip_check(hipMemcpyAsync(&o, dso.p, sizeof(o), hipMemcpyDeviceToHost, stream), "read split");
-        if (num_features) hip_check(hipMemcpyAsync(splittable, dsp.p, num_features, hipMemcpyDeviceToHost, stream), "read splittable");
         sync();
+        const SplitOut &o = h_split.p->split;
+        if (num_features) std::memcpy(splittable, h_split_flags.p + n, num_features);
         to_info(o, out);
-        if (o.found && o.rule == RULE_SORTED) {  // the rule's bins in order (split.rs:114-116)
-            uint8_t order[256];
-            hip_check(hipMemcpy(order, dorder.p + static_cast<size_t>(o.feature) * 256, 256, hipMemcpyDeviceToHost), "read categories");
-            for (uint32_t i = 0; i < o.cat_count && i < 256; ++i) out->cat_bins[i] = order[i];
-        }
+        if (o.found && o.rule == RULE_SORTED)  // the rule's bins in order (split.rs:114-116)
+            for (uint32_t i = 0; i < o.cat_count && i < 256; ++i) out->cat_bins[i] = h_split.p->order[i];
     }
 
     static void to_info(const SplitOut &o, srocm_split_info *out) {
@@ -2024,7 +2036,7 @@ struct Context {
     uint32_t child_shares(uint32_t jcap) const { return std::min<uint32_t>(CHILD_MAX, jcap + k1_groups() / CHILD_SHARE); }
     uint32_t child_rows() const { return std::min<uint32_t>(CHILD_MAX, k1_groups() / CHILD_SHARE + k1_groups() / CHILD_SPLIT + 1); }
     uint32_t nslot() const { return std::max<uint32_t>(ncgb + nwide, 1); }
-    uint32_t scan_blocks() const { return 8 * cus; }   // k_step_scan's grid: four waves a block, a wave per item
+    uint32_t scan_blocks() const { return 32 * cus; }  // k_step_scan's grid: a wave per item
     uint32_t reduce_blocks() const { return 8 * cus; } // k_step_reduce's grid
 
     void ensure_grow(uint32_t L) {
@@ -2358,9 +2370,9 @@ void Context::grow(const srocm_grow_spec &spec, HostTree &tree, std::vector<sroc
         k_root_prep<<<1, 256, 0, stream>>>(g);
         launch_check("k_root_prep");
         if (has_narrow)
-            k_split_scan<false><<<dim3(div_up(nf, 4), 1), 256, 0, stream>>>(d_jobs.p, dfeats.p, d_eval.p, nf, g.cfg, g.sg, g.sh, nullptr, g.dsc);
+            k_split_scan<false, int64_t><<<div_up(nf, 4), 256, 0, stream>>>(ScanJob{}, d_jobs.p, dfeats.p, d_eval.p, nf, g.cfg, g.sg, g.sh, nullptr, g.dsc);
         if (has_wide)
-            k_split_scan<true><<<dim3(div_up(nf, 4), 1), 256, 0, stream>>>(d_jobs.p, dfeats.p, d_eval.p, nf, g.cfg, g.sg, g.sh, nullptr, g.dsc);
+            k_split_scan<true, int64_t><<<div_up(nf, 4), 256, 0, stream>>>(ScanJob{}, d_jobs.p, dfeats.p, d_eval.p, nf, g.cfg, g.sg, g.sh, nullptr, g.dsc);
         launch_check("k_split_scan");
         if (L <= LEAVES_SMALL) k_root_select<LEAVES_SMALL><<<1, 512, 0, stream>>>(g);
         else k_root_select<GROW_MAX_LEAVES><<<1, 512, 0, stream>>>(g);
@@ -2450,7 +2462,7 @@ void Context::grow(const srocm_grow_spec &spec, HostTree &tree, std::vector<sroc
                     k_step_reduce<<<reduce_blocks(), 256, 0, stream>>>(g, ra);
                     launch_check("k_step_reduce");
                     const ScanStepArgs sca{wide_feats.p, d_plans.p + parity};
-                    k_step_scan<<<scan_blocks(), 256, 0, stream>>>(g, sca);
+                    k_step_scan<<<scan_blocks(), 64, 0, stream>>>(g, sca);
                     launch_check("k_step_scan");
                 }
                 SelectArgs sa2{d_plans.p + parity, d_plans.p + (parity ^ 1u)};
@@ -3041,11 +3053,8 @@ int srocm_gradients(void *ctx, float *grad, float *hess, size_t len) {
     return guard(ctx, [&](Context &c) {
         c.require_loaded();
         if (len != c.rows) fail(SROCM_ERR_DEVICE, "gradient buffers of " + std::to_string(len) + " values, expected " + std::to_string(c.rows));
-        if (len) {
-            hip_check(hipMemcpyAsync(grad, c.grad.p, len * 4, hipMemcpyDeviceToHost, c.stream), "read grad");
-            hip_check(hipMemcpyAsync(hess, c.hess.p, len * 4, hipMemcpyDeviceToHost, c.stream), "read hess");
-        }
-        c.sync();
+        c.copy_out(grad, c.grad.p, len * 4);
+        c.copy_out(hess, c.hess.p, len * 4);
     });
 }
 
@@ -3055,8 +3064,7 @@ int srocm_partition_rows(void *ctx, uint32_t *out, size_t len) {
         if (len > c.rows) fail(SROCM_ERR_DEVICE, "partition read of " + std::to_string(len) + " rows, the training set has " + std::to_string(c.rows));
         if (len && !out) fail(SROCM_ERR_DEVICE, "null output");
         c.ensure_order();
-        if (len) hip_check(hipMemcpyAsync(out, c.part.p, len * 4, hipMemcpyDeviceToHost, c.stream), "read partition");
-        c.sync();
+        c.copy_out(out, c.part.p, len * 4);
     });
 }
 

@@ -638,6 +638,7 @@ struct PartArgs {
     uint32_t col16, wide;  // u16 column-major bins; the split is a wide feature's numerical rule
     uint32_t *block_left;  // [grid]
     uint32_t *dev_left;    // total left count (written by block 0 of pass 2)
+    uint32_t *host_left;   // and in the host's pinned memory (or null)
     uint32_t begin, count;
     uint32_t left_bins[8];
     // bagging
@@ -707,7 +708,10 @@ __global__ __launch_bounds__(256) void k_part_scatter(PartArgs a) {
     __syncthreads();
     before = red[0][0] + red[0][1] + red[0][2] + red[0][3];
     total = red[1][0] + red[1][1] + red[1][2] + red[1][3];
-    if (blockIdx.x == 0 && tid == 0 && a.dev_left) *a.dev_left = total;
+    if (blockIdx.x == 0 && tid == 0) {
+        *a.dev_left = total;
+        if (a.host_left) *a.host_left = total;
+    }
     const uint32_t start = blockIdx.x * per_block;
     const uint32_t end = start + per_block < a.count ? start + per_block : a.count;
     uint32_t lpos = before;                    // next left slot (relative to begin)
@@ -1344,20 +1348,50 @@ __device__ __forceinline__ bool candidate_stop(const Ctx &c, const SplitCfgDev &
     return other_small && !skip;
 }
 
-// Where a scan reads a feature's units from: a histogram in memory ({g, h} i64 per bin), or a child's histogram in LDS
-// (k_step_children: g and h planes of doubles, every value an exact integer).
-struct MemUnits {
-    const int64_t *p;  // the feature's bin 0
-    __device__ __forceinline__ double g(int b) const { return static_cast<double>(p[2 * b]); }
-    __device__ __forceinline__ double h(int b) const { return static_cast<double>(p[2 * b + 1]); }
-};
+// Where a scan reads a feature's units from: planes of doubles in LDS, g and h apart, every value an exact integer.
 struct LdsUnits {
     const double *pg, *ph;
     __device__ __forceinline__ double g(int b) const { return pg[b]; }
     __device__ __forceinline__ double h(int b) const { return ph[b]; }
 };
-__device__ __forceinline__ MemUnits feature_units(const int64_t *hist, const FeatDev &m) {
-    return MemUnits{hist + 2 * static_cast<size_t>(m.hist_offset)};
+// The same with a gap each 16 bins, for the wide scan, whose lanes read bins 16 apart.
+struct PadUnits {
+    const double *pg, *ph;
+    __device__ __forceinline__ double g(int b) const { return pg[b + (b >> 4)]; }
+    __device__ __forceinline__ double h(int b) const { return ph[b + (b >> 4)]; }
+};
+
+// A wave's LDS planes of one feature's units: up to 256 bins, or 1024 (two-byte bins) with PadUnits' gaps.
+template <bool WIDE> struct UnitPlanes {
+    static constexpr int BINS = WIDE ? 1024 : 256;
+    double g[WIDE ? BINS + BINS / 16 : BINS], h[WIDE ? BINS + BINS / 16 : BINS];
+};
+// Fills them from a histogram ({g, h} per bin, in memory) with whole-line loads, all in flight together: lane l takes bins
+// l, l + 64, ... (a scan's own lanes hold 4 or 16 neighbouring bins, so reading memory by them touched a line a lane and
+// load: k_step_scan 64 -> 48 us a step on 6M x 32 two-byte bins). T: int64_t, or double for a histogram of the host's.
+// Within the wave.
+template <bool WIDE, class T>
+__device__ __forceinline__ auto stage_units(const T *hist, const FeatDev &m, UnitPlanes<WIDE> &pl) {
+    struct alignas(16) Pair {
+        T g, h;
+    };
+    const uint32_t lane = threadIdx.x & 63u;
+    const Pair *p = reinterpret_cast<const Pair *>(hist) + m.hist_offset;
+    const uint32_t nb = m.num_bins;
+    constexpr int N = UnitPlanes<WIDE>::BINS / 64;
+    Pair v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = p[min(lane + 64u * i, nb ? nb - 1u : 0u)];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const uint32_t b = lane + 64u * i, at = WIDE ? b + (b >> 4) : b;
+        pl.g[at] = static_cast<double>(static_cast<int64_t>(v[i].g));
+        pl.h[at] = static_cast<double>(static_cast<int64_t>(v[i].h));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if constexpr (WIDE) return PadUnits{pl.g, pl.h};
+    else return LdsUnits{pl.g, pl.h};
 }
 
 constexpr uint32_t UNIT_FEATS = 16;  // features a scan unit holds at most (segments of 4 lanes)
@@ -1447,11 +1481,10 @@ __device__ __forceinline__ double seg_max_f64(double v) {  // v is never NaN
 // 16l .. 16l + 15. The same candidates, stops and ties as scan_numerical, in two passes over the lane's bins so that
 // only the units stay in registers: the first finds both directions' stops, the second evaluates the candidates in
 // range, re-forming the exact prefix sums as it goes.
-__device__ void scan_numerical_wide(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const int64_t *hist,
-                                    bool &rf, Grown &rg, bool &ff, Grown &fg) {
+__device__ __forceinline__ void scan_numerical_wide(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const PadUnits &u,
+                                                    bool &rf, Grown &rg, bool &ff, Grown &fg) {
     constexpr int NPB = 16;
     const int lane = static_cast<int>(threadIdx.x & 63u);
-    const int64_t *h = hist + 2 * static_cast<size_t>(m.hist_offset);
     const int nb = static_cast<int>(m.num_bins);
     const bool two = scan_two_way(m);
     const int top = two ? nb - 2 : nb - 1;
@@ -1460,8 +1493,8 @@ __device__ void scan_numerical_wide(const Ctx &c, const SplitCfgDev &cfg, const 
     for (int j = 0; j < NPB; ++j) {
         const int b = NPB * lane + j;
         const int t = b <= top ? b : 0;
-        gu[j] = b <= top ? static_cast<double>(h[2 * t]) : 0.0;
-        hu[j] = b <= top ? static_cast<double>(h[2 * t + 1]) : 0.0;
+        gu[j] = b <= top ? u.g(t) : 0.0;
+        hu[j] = b <= top ? u.h(t) : 0.0;
     }
     // per-bin counts (split.rs:196-198): `(x + 0.5) as i64`
     auto count_of = [&](int j) {
@@ -2075,70 +2108,49 @@ __device__ __forceinline__ FeatCand categorical_candidate(const Ctx &c, const Sp
     return sorted_scan(c, cfg, m, u, sc, order_out);
 }
 
-// split.rs:584-620 find_numerical (or a categorical search) for one feature of one leaf, by one wave. WIDE: the
-// feature has two-byte bins (numerical, up to 1024); the kernels that scan them are instantiated apart, so the
-// wide scan's registers do not lower the occupancy of the byte-bin scan.
-template <bool WIDE>
-__device__ FeatCand scan_feature(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const int64_t *hist, bool evaluate,
-                                 CatScratch &sc, uint8_t *order_out) {
-    if (!scan_searched(c, m, evaluate)) return FeatCand{};
-    Grown rg = {}, fg = {};
-    bool rf, ff;
-    if constexpr (WIDE) {
-        scan_numerical_wide(c, cfg, m, hist, rf, rg, ff, fg);
-    } else {
-        const MemUnits u = feature_units(hist, m);
-        if (m.kind == 2) return categorical_candidate(c, cfg, m, u, sc, order_out);
-        scan_numerical(c, cfg, m, u, rf, rg, ff, fg);
-    }
-    return feature_candidate(c, m, rf, rg, ff, fg);
-}
-
-// grid: (ceil(num_features / 4), num_jobs); 4 waves per block, a wave per feature.
-template <bool WIDE>
-__global__ __launch_bounds__(256) void k_split_scan(const ScanJob *__restrict__ jobs, const FeatDev *__restrict__ feats,
+// split.rs:919-961 over one leaf's histogram, a wave a feature: split.rs:584-620 find_numerical, or a categorical search.
+// WIDE: the features of two-byte bins (numerical, up to 1024), in an instance of their own, so the wide scan's registers do
+// not lower the occupancy of the byte-bin scan. T: the histogram's units, int64_t, or double (a histogram of the host's,
+// read where the host put it). One wave a feature whatever its bins: all of a leaf's features are on the chip at once.
+// `from`, when set, holds the job (made on the device). grid: ceil(num_features / 4); 256 threads.
+template <bool WIDE, class T>
+__global__ __launch_bounds__(256) void k_split_scan(ScanJob given, const ScanJob *from, const FeatDev *__restrict__ feats,
                                                     const uint8_t *__restrict__ evaluate, uint32_t num_features,
                                                     SplitCfgDev cfg, double sg, double sh,
                                                     uint8_t *cat_order /* [feature][256] or null */,
-                                                    const DevScales *dsc /* when set: the scales */,
-                                                    const uint8_t *skip = nullptr /* features k_split_scan_seg takes */) {
+                                                    const DevScales *dsc /* when set: the scales */) {
+    __shared__ UnitPlanes<WIDE> planes[4];
+    __shared__ __align__(16) uint8_t cats[WIDE ? 16 : 4 * sizeof(CatScratch)];
+    const uint32_t wave = threadIdx.x >> 6, f = blockIdx.x * 4 + wave;
+    if (f >= num_features) return;
+    const FeatDev m = feats[f];
+    const bool ev = evaluate[f] != 0;
+    const ScanJob job = from ? *from : given;
     if (dsc) {
         sg = dsc->sg;
         sh = dsc->sh;
     }
-    __shared__ CatScratch cats[4];
-    const ScanJob &job = jobs[blockIdx.y];
-    uint32_t f = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (f >= num_features || (feats[f].wide != 0) != WIDE) return;  // the other instantiation's feature
-    if (skip && skip[f]) return;
-    Ctx c = make_ctx(cfg, sg, sh, job.units_grad, job.units_hess, job.count);
-    FeatCand r = scan_feature<WIDE>(c, cfg, feats[f], job.hist, evaluate[f] != 0, cats[threadIdx.x >> 6],
-                              cat_order ? cat_order + static_cast<size_t>(f) * 256 : nullptr);
-    if ((threadIdx.x & 63) == 0) job.out[f] = r;
-}
-
-// k_split_scan for scan units of several numerical byte features of at most 64 bins (16 or 4 lanes a feature, as in
-// k_step_children): unit u holds unit_feat[u * UNIT_FEATS ...] (-1 padding), unit_segl[u] lanes each. A wave per
-// unit and job. grid: (ceil(units / 4), jobs), 256 threads.
-__global__ __launch_bounds__(256) void k_split_scan_seg(const ScanJob *__restrict__ jobs, const FeatDev *__restrict__ feats,
-                                                        const uint8_t *__restrict__ evaluate, const int32_t *unit_feat,
-                                                        const uint32_t *unit_segl, uint32_t num_units, SplitCfgDev cfg,
-                                                        double sg, double sh) {
-    const ScanJob &job = jobs[blockIdx.y];
-    const uint32_t u = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
-    if (u >= num_units) return;
-    const uint32_t segl = unit_segl[u];  // 16 or 4, wave-uniform
-    const int32_t f = unit_feat[u * UNIT_FEATS + lane / segl];
-    const FeatDev m = f >= 0 ? feats[f] : FeatDev{};
+    if ((m.wide != 0) != WIDE) return;  // the other instance's feature
     const Ctx c = make_ctx(cfg, sg, sh, job.units_grad, job.units_hess, job.count);
-    Grown rg = {}, fg = {};
-    bool rf = false, ff = false;
-    const MemUnits units = feature_units(job.hist, m);
-    if (segl == 16u) scan_numerical<16>(c, cfg, m, units, rf, rg, ff, fg);
-    else scan_numerical<4>(c, cfg, m, units, rf, rg, ff, fg);
     FeatCand r = {};
-    if (f >= 0 && scan_searched(c, m, evaluate[f] != 0)) r = feature_candidate(c, m, rf, rg, ff, fg);
-    if ((lane & (segl - 1u)) == 0 && f >= 0) job.out[f] = r;
+    if (scan_searched(c, m, ev)) {
+        const auto u = stage_units<WIDE>(reinterpret_cast<const T *>(job.hist), m, planes[wave]);
+        if constexpr (WIDE) {
+            Grown rg = {}, fg = {};
+            bool rf, ff;
+            scan_numerical_wide(c, cfg, m, u, rf, rg, ff, fg);
+            r = feature_candidate(c, m, rf, rg, ff, fg);
+        } else if (m.kind == 2) {
+            r = categorical_candidate(c, cfg, m, u, reinterpret_cast<CatScratch *>(cats)[wave],
+                                      cat_order ? cat_order + static_cast<size_t>(f) * 256 : nullptr);
+        } else {
+            Grown rg = {}, fg = {};
+            bool rf, ff;
+            scan_numerical(c, cfg, m, u, rf, rg, ff, fg);
+            r = feature_candidate(c, m, rf, rg, ff, fg);
+        }
+    }
+    if ((threadIdx.x & 63) == 0) job.out[f] = r;
 }
 
 // The leaf's SplitInfo (split.rs:631-651 finish) and splittable flags from the per-feature candidates: the
@@ -2235,11 +2247,29 @@ __device__ void select_split(const ScanJob &job, int64_t count, uint32_t num_fea
     __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void k_split_select(const ScanJob *__restrict__ jobs, uint32_t num_features,
-                                                      SplitCfgDev cfg, double sg, double sh, SplitOut *out,
-                                                      uint8_t *splittable /* [job][num_features] */) {
-    const ScanJob &job = jobs[blockIdx.x];
-    select_split(job, job.count, num_features, cfg, sg, sh, out + blockIdx.x, splittable + (size_t)blockIdx.x * num_features);
+// The trait's split search's end: the leaf's SplitOut, its splittable flags and, for a sorted categorical rule, its bins in
+// order, written where the host reads them. One block.
+__global__ __launch_bounds__(256) void k_split_select(ScanJob job, uint32_t num_features, SplitCfgDev cfg, double sg, double sh,
+                                                      const uint8_t *cat_order, SplitOut *out, uint8_t *order_out,
+                                                      uint8_t *splittable) {
+    __shared__ SplitOut o;
+    select_split(job, job.count, num_features, cfg, sg, sh, &o, splittable);
+    __syncthreads();
+    static_assert(sizeof(SplitOut) % 4 == 0 && sizeof(SplitOut) / 4 <= 256, "a split copies in one pass");
+    if (threadIdx.x < sizeof(SplitOut) / 4)
+        reinterpret_cast<uint32_t *>(out)[threadIdx.x] = reinterpret_cast<const uint32_t *>(&o)[threadIdx.x];
+    if (o.found && o.rule == RULE_SORTED) order_out[threadIdx.x] = cat_order[static_cast<size_t>(o.feature) * 256 + threadIdx.x];
+}
+
+// A histogram's units as the doubles the trait returns, and a partition's left count (when given), written to the host's
+// pinned memory. A thread a bin.
+__global__ __launch_bounds__(256) void k_hist_to_host(const int64_t *__restrict__ hist, double *__restrict__ out, uint64_t bins,
+                                                      const uint32_t *left, uint32_t *left_out) {
+    if (left && blockIdx.x == 0 && threadIdx.x == 0) *left_out = *left;
+    for (uint64_t b = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; b < bins; b += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
+        const longlong2 v = reinterpret_cast<const longlong2 *>(hist)[b];
+        reinterpret_cast<double2 *>(out)[b] = make_double2(static_cast<double>(v.x), static_cast<double>(v.y));
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -5033,12 +5063,14 @@ __global__ __launch_bounds__(256) void k_step_reduce(GrowState g, ReduceStepArgs
 
 // Scan items (job, two-byte feature, child), a wave each in a grid-stride loop: the feature scanned in both directions
 // (split.rs:584-620) over the child's histogram (the built one, or the sibling k_step_reduce formed in the parent's slot)
-// and its candidate written to its own slot. grid: any, 256 threads.
-__global__ __launch_bounds__(256) void k_step_scan(GrowState g, ScanStepArgs a) {
+// and its candidate written to its own slot. A wave a block: the planes of four would leave one block a compute unit.
+// grid: any, 64 threads.
+__global__ __launch_bounds__(64) void k_step_scan(GrowState g, ScanStepArgs a) {
+    __shared__ UnitPlanes<true> planes;
     const StepPlan &P = *a.plan;  // empty once the tree is done (k_step_select)
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t total = P.total_scan * 2u;  // scan items count features: a wave per feature and child
-    for (uint32_t item = blockIdx.x * 4u + (threadIdx.x >> 6); item < total; item += gridDim.x * 4u) {
+    for (uint32_t item = blockIdx.x; item < total; item += gridDim.x) {
         const uint32_t gi = item >> 1, child = item & 1u;
         const uint32_t j = job_of(P.scan_base, P.njobs, gi);
         const JobPlan &J = P.jobs[j];
@@ -5053,7 +5085,7 @@ __global__ __launch_bounds__(256) void k_step_scan(GrowState g, ScanStepArgs a) 
         if (scan_searched(c, sm, sev)) {
             Grown rg = {}, fg = {};
             bool rf, ff;
-            scan_numerical_wide(c, g.cfg, sm, hist, rf, rg, ff, fg);
+            scan_numerical_wide(c, g.cfg, sm, stage_units<true>(hist, sm, planes), rf, rg, ff, fg);
             r = feature_candidate(c, sm, rf, rg, ff, fg);
         }
         if (lane == 0) {
