@@ -66,9 +66,9 @@ def kernel_key(name):
 def timed_window(rows, warmup, steps):
     """The dispatch records of the timed iterations (after `warmup` iterations, `steps` of them) of a run of this
     script. An iteration starts after the previous tree's score update (k_add_leaf_values) that precedes its tree's
-    k_grow_init, so a window begins with an iteration's gradients. `rows` are rocprofv3 CSV records in dispatch
+    k_root_select, so a window begins with an iteration's gradients. `rows` are rocprofv3 CSV records in dispatch
     order."""
-    starts = [i for i, r in enumerate(rows) if kernel_key(r["Kernel_Name"]).startswith("k_grow_init")]
+    starts = [i for i, r in enumerate(rows) if kernel_key(r["Kernel_Name"]).startswith("k_root_select")]
     if warmup < 1 or len(starts) < warmup + steps:
         raise SystemExit(f"the profile holds {len(starts)} trees; a window of {steps} after {warmup} warm-up "
                          "iterations (at least one) needs more")

@@ -390,8 +390,11 @@ struct Context {
     std::vector<float> h_label_v, h_weight_v;
     DevBuf<int32_t> packed, partial;
     DevBuf<uint32_t> part, part2, block_left, scalars;
-    DevBuf<uint32_t> maxima;  // the gradient maxima, MAX_SLOTS pairs
-    bool maxima_clear = false; // maxima holds zeros on the stream (k_quant_spec cleared it after reading)
+    DevBuf<uint32_t> maxima;   // the gradient maxima, MAX_SLOTS pairs, twice: the boosting loop's iterations take turns
+    uint32_t maxima_at = 0;    // the half the next gradients take
+    bool maxima_clear = false; // which holds zeros on the stream (k_quantize_dev cleared it while it read the other)
+    uint32_t *maxima_now() const { return maxima.p + 2 * MAX_SLOTS * maxima_at; }
+    bool codes_ready = false;  // codes0 holds the rows' codes in row order (k_quantize_dev), for the next grown tree
     DevBuf<uint8_t> codes0, codes1;  // grown trees: each row's gradient code beside its id in part / part2
     DevBuf<FeatDev> dfeats;
     DevBuf<ColGroup> d_cgs;
@@ -423,7 +426,7 @@ struct Context {
     DevBuf<double> d_leaf_vw;           // per tree of a boosting call (2 GROW_MAX_LEAVES + 1 each): its renewed leaf
                                         // values, then (from GROW_MAX_LEAVES) weights, then the gate
     DevBuf<uint32_t> d_gate;            // the boosted tree's leaves once it is complete with a split (k_tree_nodes)
-    DevBuf<DevScales> d_scales;         // the boosting loop's quantization, made on the device (k_quant_spec)
+    DevBuf<DevScales> d_scales;         // the boosting loop's quantization, made on the device (k_quantize_dev)
     const DevScales *grow_dsc = nullptr;  // set while the boosting loop grows: the scales of GrowState
     hipEvent_t tree_event = nullptr;    // a grown tree's readback has landed
     hipEvent_t steps_event = nullptr;   // a batch of split steps has ended (the readback waits for it)
@@ -689,7 +692,7 @@ struct Context {
             launch_check("k_rank_scale");
             rank_flag_pending = mode >= RANK_FACTOR_DEVICE;
         }
-        k_max_abs<<<grid_rows(rows), 256, 0, stream>>>(grad.p, hess.p, rows, maxima.p);
+        k_max_abs<<<grid_rows(rows), 256, 0, stream>>>(grad.p, hess.p, rows, maxima_now());
         launch_check("k_max_abs");
         rank_flag_queued = false;  // queue_rank_flag copies it, once the kernels after these are queued
     }
@@ -775,7 +778,7 @@ struct Context {
         build_slabs();
         // device buffers
         scalars.alloc(16);
-        maxima.alloc(2 * MAX_SLOTS);
+        maxima.alloc(4 * MAX_SLOTS);
         maxima_clear = false;
         hip_check(hipMemsetAsync(scalars.p + 15, 0, 4, stream), "zero bin check");
         train = DevData{};
@@ -1254,7 +1257,7 @@ struct Context {
     // ------------------------------------------------------------------------------------------------
 
     std::pair<double, double> read_maxima() {
-        hip_check(hipMemcpyAsync(h_u32.p, maxima.p, 8 * MAX_SLOTS, hipMemcpyDeviceToHost, stream), "read maxima");
+        hip_check(hipMemcpyAsync(h_u32.p, maxima_now(), 8 * MAX_SLOTS, hipMemcpyDeviceToHost, stream), "read maxima");
         sync();
         uint32_t ug = 0, uh = 0;
         for (uint32_t k = 0; k < MAX_SLOTS; ++k) {
@@ -1277,9 +1280,9 @@ struct Context {
         if (n != rows) fail(SROCM_ERR_DEVICE, "gradient arrays of " + std::to_string(n) + " rows, expected " + std::to_string(rows));
         hip_check(hipMemcpyAsync(grad.p, g, n * 4, hipMemcpyHostToDevice, stream), "upload grad");
         hip_check(hipMemcpyAsync(hess.p, h, n * 4, hipMemcpyHostToDevice, stream), "upload hess");
-        hip_check(hipMemsetAsync(maxima.p, 0, 8 * MAX_SLOTS, stream), "zero maxima");
+        hip_check(hipMemsetAsync(maxima_now(), 0, 8 * MAX_SLOTS, stream), "zero maxima");
         maxima_clear = false;
-        k_max_abs<<<grid_rows(n), 256, 0, stream>>>(grad.p, hess.p, n, maxima.p);
+        k_max_abs<<<grid_rows(n), 256, 0, stream>>>(grad.p, hess.p, n, maxima_now());
         launch_check("k_max_abs");
         return read_maxima();
     }
@@ -1314,8 +1317,12 @@ struct Context {
                                             std::to_string(wg) + " rows per histogram workgroup could overflow its 32-bit sums");
     }
 
+    // units that travel as one-byte codes beside the row ids (packed_code)
+    bool units_fit_codes(int64_t gq, int64_t hq) const { return !q32 && gq <= CODE_MAX_G && hq <= CODE_MAX_H; }
+
     void quantize(const srocm_quant_spec &s) {
         require_loaded();
+        codes_ready = false;
         check_quant_units(s.grad_max_q, s.hess_max_q);
         set_mode(q32_for(s.grad_max_q, s.hess_max_q), std::max(s.grad_max_q, s.hess_max_q));
         QuantDev q{s.inv_grad_scale, s.inv_hess_scale, s.grad_max_q, s.hess_max_q, s.constant_hessian, s.stochastic, s.seed, s.iteration};
@@ -1328,15 +1335,19 @@ struct Context {
         quantized_once = true;
     }
 
-    uint32_t reset_partition(const srocm_bag &bag) {
+    // `written`: the partition is queued to hold every row in order already.
+    uint32_t reset_partition(const srocm_bag &bag, bool written = false) {
         require_loaded();
         pending_order.on = false;  // the partition is rewritten
         if (rows == 0) {
             part_len = 0;
             return 0;
         }
-        k_iota<<<grid_rows(rows), 256, 0, stream>>>(part.p, rows);
-        launch_check("k_iota");
+        if (!written) {
+            codes_ready = false;
+            k_iota<<<grid_rows(rows), 256, 0, stream>>>(part.p, rows);
+            launch_check("k_iota");
+        }
         if (bag.kind == SROCM_BAG_ALL) {
             part_len = static_cast<uint32_t>(rows);
             return part_len;
@@ -1951,8 +1962,8 @@ struct Context {
         const ScanJob job{reinterpret_cast<const int64_t *>(hist), sums.grad, sums.hess, sums.count, split_cands.p};
         uint8_t *order = cats ? split_order.p : nullptr;
         const uint32_t grid = div_up(num_features, 4);
-        if (narrow) k_split_scan<false, T><<<grid, 256, 0, stream>>>(job, nullptr, split_feats.p, h_split_flags.p, num_features, cfg_dev(cfg), sg, sh, order, nullptr);
-        if (wide) k_split_scan<true, T><<<grid, 256, 0, stream>>>(job, nullptr, split_feats.p, h_split_flags.p, num_features, cfg_dev(cfg), sg, sh, order, nullptr);
+        if (narrow) k_split_scan<false, T><<<grid, 256, 0, stream>>>(job, split_feats.p, h_split_flags.p, num_features, cfg_dev(cfg), sg, sh, order);
+        if (wide) k_split_scan<true, T><<<grid, 256, 0, stream>>>(job, split_feats.p, h_split_flags.p, num_features, cfg_dev(cfg), sg, sh, order);
         launch_check("k_split_scan");
         k_split_select<<<1, 256, 0, stream>>>(job, num_features, cfg_dev(cfg), sg, sh, order, &h_split.p->split, h_split.p->order, h_split_flags.p + n);
         launch_check("k_split_select");
@@ -1994,7 +2005,7 @@ struct Context {
     DevBuf<TLeaf> d_tl;               // the speculative tree's leaves
     DevBuf<TKey> d_tk;
     DevBuf<uint8_t> d_leaf_left;
-    DevBuf<uint8_t> d_splittable, d_eval, d_mask;
+    DevBuf<uint8_t> d_splittable, d_mask;
     std::vector<uint8_t> d_mask_host;  // what d_mask holds (empty: unknown), so an unchanged mask is not uploaded again
     DevBuf<ScanJob> d_jobs;
     DevBuf<FeatCand> d_root_cands, d_cands;
@@ -2048,7 +2059,6 @@ struct Context {
         d_tk.alloc(tcap);
         d_leaf_left.alloc(L);
         d_splittable.alloc(static_cast<size_t>(tcap) * nf);
-        d_eval.alloc(nf);
         d_mask.alloc(nf);
         d_mask_host.clear();
         d_jobs.alloc(1);
@@ -2105,7 +2115,6 @@ struct Context {
         g.cands = d_cands.p;
         g.cand_gain = d_cand_gain.p;
         g.cand_feat = d_cand_feat.p;
-        g.evaluate = d_eval.p;
         g.mask = d_mask.p;
         g.feats = dfeats.p;
         g.tree = TreeDev{reinterpret_cast<int32_t *>(tp + tl.sf), reinterpret_cast<uint32_t *>(tp + tl.tb), tp + tl.dl,
@@ -2290,16 +2299,16 @@ std::pair<double, double> Context::compute_gradients() {
 void Context::launch_gradients(bool host_factors) {
     require_loaded();
     rank_flag_pending = false;
-    if (!maxima_clear) hip_check(hipMemsetAsync(maxima.p, 0, 8 * MAX_SLOTS, stream), "zero maxima");
+    if (!maxima_clear) hip_check(hipMemsetAsync(maxima_now(), 0, 8 * MAX_SLOTS, stream), "zero maxima");
     maxima_clear = false;
     if (rows && objective == SROCM_OBJ_LAMBDARANK) {
         ranking_gradients(host_factors);
     } else if (rows) {
         const float *w = has_weight ? weight.p : nullptr;
         if (objective == SROCM_OBJ_REGRESSION)
-            k_grad_regression<<<grid_rows(rows), 256, 0, stream>>>(train.scores.p, label.p, w, grad.p, hess.p, rows, maxima.p);
+            k_grad_regression<<<grid_rows(rows), 256, 0, stream>>>(train.scores.p, label.p, w, grad.p, hess.p, rows, maxima_now());
         else
-            k_grad_binary<<<grid_rows(rows), 256, 0, stream>>>(train.scores.p, label.p, w, grad.p, hess.p, rows, sigmoid, maxima.p);
+            k_grad_binary<<<grid_rows(rows), 256, 0, stream>>>(train.scores.p, label.p, w, grad.p, hess.p, rows, sigmoid, maxima_now());
         launch_check("k_grad");
     }
 }
@@ -2340,18 +2349,23 @@ void Context::grow(const srocm_grow_spec &spec, HostTree &tree, std::vector<sroc
         hip_check(hipMemcpyAsync(d_mask.p, h_stage.p, nf, hipMemcpyHostToDevice, stream), "upload mask");
         d_mask_host = mask;
     }
-    k_grow_init<<<1, 64, 0, stream>>>(g, spec.root.begin, spec.root.count, spec.root_count, root_searched ? 1u : 0u);
-    launch_check("k_grow_init");
+    if (!root_searched) {
+        k_grow_init<<<1, 64, 0, stream>>>(g, spec.root.begin, spec.root.count, spec.root_count);
+        launch_check("k_grow_init");
+    }
     // small units travel beside the row ids as one-byte codes (packed_code), so the split steps' histograms read them
     // with the rows instead of gathering the packed words
-    const bool codes = !q32 && max_gq <= CODE_MAX_G && max_hq <= CODE_MAX_H && root_searched && spec.root.count;
+    const bool codes = units_fit_codes(max_gq, max_hq) && root_searched && spec.root.count;
     if (codes) {
         codes0.alloc(rows);
         codes1.alloc(rows);
-        k_gh_codes<<<std::min<uint32_t>(div_up(spec.root.count, 256), cus * 8), 256, 0, stream>>>(
-            part.p, packed.p, spec.root.begin, spec.root.count, codes0.p);
-        launch_check("k_gh_codes");
+        if (!codes_ready) {
+            k_gh_codes<<<std::min<uint32_t>(div_up(spec.root.count, 256), cus * 8), 256, 0, stream>>>(
+                part.p, packed.p, spec.root.begin, spec.root.count, codes0.p);
+            launch_check("k_gh_codes");
+        }
     }
+    codes_ready = false;  // the tree's steps move them
     const HistUse used_root = hist_use([&](uint32_t f) { return mask[f] || static_cast<int32_t>(f) == sums_feature; });
     // the tree block comes back with every check for the end of the tree
     const TreeLayout &lay = tree_layout;
@@ -2367,13 +2381,10 @@ void Context::grow(const srocm_grow_spec &spec, HostTree &tree, std::vector<sroc
     if (root_searched) {
         // the root histogram goes into slot 0
         launch_hist(spec.root.begin, spec.root.count, nullptr, 0, pool.p, nullptr, used_root);
-        k_root_prep<<<1, 256, 0, stream>>>(g);
-        launch_check("k_root_prep");
-        if (has_narrow)
-            k_split_scan<false, int64_t><<<div_up(nf, 4), 256, 0, stream>>>(ScanJob{}, d_jobs.p, dfeats.p, d_eval.p, nf, g.cfg, g.sg, g.sh, nullptr, g.dsc);
+        if (has_narrow) k_root_scan<false><<<div_up(nf, 4), 256, 0, stream>>>(g, spec.root.begin, spec.root.count, spec.root_count, 1u);
         if (has_wide)
-            k_split_scan<true, int64_t><<<div_up(nf, 4), 256, 0, stream>>>(ScanJob{}, d_jobs.p, dfeats.p, d_eval.p, nf, g.cfg, g.sg, g.sh, nullptr, g.dsc);
-        launch_check("k_split_scan");
+            k_root_scan<true><<<div_up(nf, 4), 256, 0, stream>>>(g, spec.root.begin, spec.root.count, spec.root_count, has_narrow ? 0u : 1u);
+        launch_check("k_root_scan");
         if (L <= LEAVES_SMALL) k_root_select<LEAVES_SMALL><<<1, 512, 0, stream>>>(g);
         else k_root_select<GROW_MAX_LEAVES><<<1, 512, 0, stream>>>(g);
         launch_check("k_root_select");
@@ -2768,20 +2779,6 @@ uint32_t Context::boost(const srocm_train_params &p, uint32_t first, uint32_t co
         // quantize.rs:56-84 on the device: nothing waits for the gradient maxima
         launch_gradients(host_factors);
         d_scales.alloc(1);
-        k_quant_spec<<<1, MAX_SLOTS, 0, stream>>>(maxima.p, d_scales.p, p.num_grad_quant_bins, constant_hessian ? 1u : 0u, 1.0,
-                                           p.stochastic_rounding != 0 ? 1u : 0u, p.data_random_seed, it);
-        launch_check("k_quant_spec");
-        maxima_clear = true;
-        if (rows) {
-            k_quantize_dev<<<grid_rows(rows), 256, 0, stream>>>(grad.p, hess.p, packed.p, rows, row_offset, d_scales.p);
-            launch_check("k_quantize");
-        }
-        queue_rank_flag();
-        max_gq = static_cast<int64_t>(p.num_grad_quant_bins / 2);
-        max_hq = static_cast<int64_t>(p.num_grad_quant_bins);
-        quantized_once = true;
-        const bool bias = trees_added == 0 && init_score_value != 0.0;
-        const bool renew = p.quant_train_renew_leaf != 0;
         srocm_bag bag{};
         if (p.bagging_fraction < 1.0 && p.bagging_freq > 0) {
             bag.kind = SROCM_BAG_BERNOULLI;
@@ -2789,7 +2786,25 @@ uint32_t Context::boost(const srocm_train_params &p, uint32_t first, uint32_t co
             bag.round = it / p.bagging_freq;
             bag.fraction = p.bagging_fraction;
         }
-        uint32_t local_rows = reset_partition(bag);
+        // without a bag the quantization writes the partition and the gradient codes too (rows in order)
+        const bool whole = bag.kind == SROCM_BAG_ALL;
+        pending_order.on = false;  // the partition is rewritten
+        codes_ready = whole && units_fit_codes(p.num_grad_quant_bins / 2, p.num_grad_quant_bins);
+        if (codes_ready) codes0.alloc(rows);
+        const SpecArgs spec{p.num_grad_quant_bins, constant_hessian ? 1u : 0u, 1.0, p.stochastic_rounding != 0 ? 1u : 0u, p.data_random_seed, it};
+        k_quantize_dev<<<std::min<uint32_t>(std::max<uint32_t>(div_up(rows, 1024), 1), cus * 8), 256, 0, stream>>>(
+            grad.p, hess.p, packed.p, rows, row_offset, maxima_now(), maxima.p + 2 * MAX_SLOTS * (maxima_at ^ 1u), d_scales.p, spec,
+            whole ? part.p : nullptr, codes_ready ? codes0.p : nullptr);
+        launch_check("k_quantize");
+        maxima_at ^= 1u;
+        maxima_clear = true;
+        queue_rank_flag();
+        max_gq = static_cast<int64_t>(p.num_grad_quant_bins / 2);
+        max_hq = static_cast<int64_t>(p.num_grad_quant_bins);
+        quantized_once = true;
+        const bool bias = trees_added == 0 && init_score_value != 0.0;
+        const bool renew = p.quant_train_renew_leaf != 0;
+        uint32_t local_rows = reset_partition(bag, whole);
         feature_mask(feats, p.feature_fraction, p.feature_fraction_seed, it, mask);
         srocm_grow_spec gs{};
         gs.cfg = p.cfg;

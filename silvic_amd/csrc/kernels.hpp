@@ -129,42 +129,77 @@ __device__ __forceinline__ float fixed_point_scale_d(double max_abs) {
     return __builtin_ldexpf(1.0f, e);
 }
 
-// One wave (launched with MAX_SLOTS threads): lane l reads slot pair l of the maxima and clears it, so the next
-// gradients' maxima start from zero without a fill of their own.
-__global__ void k_quant_spec(uint32_t *maxima, DevScales *out, uint32_t num_bins, uint32_t constant_hessian,
-                             double constant, uint32_t stochastic, uint32_t seed, uint32_t iteration) {
-    uint32_t ug = maxima[2u * threadIdx.x], uh = maxima[2u * threadIdx.x + 1u];
-    maxima[2u * threadIdx.x] = 0u;
-    maxima[2u * threadIdx.x + 1u] = 0u;
-    for (int o = 32; o >= 1; o >>= 1) {
-        const uint32_t x = __shfl_xor(ug, o), y = __shfl_xor(uh, o);
-        ug = ug > x ? ug : x;
-        uh = uh > y ? uh : y;
-    }
-    static_assert(MAX_SLOTS == 64, "one slot pair a lane");
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const double mg = static_cast<double>(__uint_as_float(ug)), mh = static_cast<double>(__uint_as_float(uh));
+// What an iteration's quantization is made from besides the gradient maxima.
+struct SpecArgs {
+    uint32_t num_bins, constant_hessian;
+    double constant;
+    uint32_t stochastic, seed, iteration;
+};
+__device__ __forceinline__ DevScales make_scales(uint32_t max_g, uint32_t max_h, const SpecArgs &a) {
+    const double mg = static_cast<double>(__uint_as_float(max_g)), mh = static_cast<double>(__uint_as_float(max_h));
     DevScales d;
-    d.q.grad_max_q = static_cast<int32_t>(num_bins / 2);
-    d.q.hess_max_q = static_cast<int32_t>(num_bins);
+    d.q.grad_max_q = static_cast<int32_t>(a.num_bins / 2);
+    d.q.hess_max_q = static_cast<int32_t>(a.num_bins);
     d.sg = positive_or_one_d(mg / static_cast<double>(d.q.grad_max_q));
-    d.sh = constant_hessian ? positive_or_one_d(constant) : positive_or_one_d(mh / static_cast<double>(d.q.hess_max_q));
+    d.sh = a.constant_hessian ? positive_or_one_d(a.constant) : positive_or_one_d(mh / static_cast<double>(d.q.hess_max_q));
     d.q.inv_grad_scale = static_cast<float>(1.0 / d.sg);
     d.q.inv_hess_scale = static_cast<float>(1.0 / d.sh);
-    d.q.constant_hessian = constant_hessian;
-    d.q.stochastic = stochastic;
-    d.q.seed = seed;
-    d.q.iteration = iteration;
+    d.q.constant_hessian = a.constant_hessian;
+    d.q.stochastic = a.stochastic;
+    d.q.seed = a.seed;
+    d.q.iteration = a.iteration;
     d.gsc = fixed_point_scale_d(mg);
     d.hsc = fixed_point_scale_d(mh);
-    *out = d;
+    return d;
 }
 
-__global__ void k_quantize_dev(const float *__restrict__ grad, const float *__restrict__ hess, int32_t *__restrict__ packed,
-                               uint64_t n, uint64_t row_offset, const DevScales *sc) {
-    const QuantDev spec = sc->q;
-    for (uint64_t r = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; r < n; r += (uint64_t)gridDim.x * blockDim.x)
-        packed[r] = quantize_row(spec, grad[r], hess[r], row_offset + r);
+// The boosting loop's quantization in one pass: every block makes the scales from the maxima (MAX_SLOTS pairs), block 0
+// leaves them for the kernels after it and clears the other gradients' maxima (`clear`: the two buffers take turns, so
+// the next gradients start from zero without a fill); then each row's packed word and, when given, the partition in row
+// order (`part`) and the rows' gradient codes (`codes`, packed_code). Bound by memory: 8 B read and 4 to 9 B written a row,
+// four rows a thread a load. Four launches before (scales, words, row ids, codes): 60 us at 10M rows, 36 now; on small
+// tables it is the three launches that count.
+__global__ __launch_bounds__(256) void k_quantize_dev(const float *__restrict__ grad, const float *__restrict__ hess,
+                                                      int32_t *__restrict__ packed, uint64_t n, uint64_t row_offset,
+                                                      const uint32_t *maxima, uint32_t *clear, DevScales *out, SpecArgs a,
+                                                      uint32_t *__restrict__ part, uint8_t *__restrict__ codes) {
+    __shared__ QuantDev s_q;
+    static_assert(MAX_SLOTS == 64, "one slot pair a lane");
+    if (threadIdx.x < MAX_SLOTS) {
+        uint32_t ug = maxima[2u * threadIdx.x], uh = maxima[2u * threadIdx.x + 1u];
+        for (int o = 32; o >= 1; o >>= 1) {
+            const uint32_t x = __shfl_xor(ug, o), y = __shfl_xor(uh, o);
+            ug = ug > x ? ug : x;
+            uh = uh > y ? uh : y;
+        }
+        const DevScales d = make_scales(ug, uh, a);
+        if (threadIdx.x == 0) s_q = d.q;
+        if (blockIdx.x == 0) {
+            clear[2u * threadIdx.x] = 0u;
+            clear[2u * threadIdx.x + 1u] = 0u;
+            if (threadIdx.x == 0) *out = d;
+        }
+    }
+    __syncthreads();
+    const QuantDev spec = s_q;
+    const uint64_t quads = n / 4;
+    for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < quads; i += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
+        const float4 g = reinterpret_cast<const float4 *>(grad)[i], h = reinterpret_cast<const float4 *>(hess)[i];
+        const uint64_t r = row_offset + 4 * i;
+        const int4 w = make_int4(quantize_row(spec, g.x, h.x, r), quantize_row(spec, g.y, h.y, r + 1),
+                                 quantize_row(spec, g.z, h.z, r + 2), quantize_row(spec, g.w, h.w, r + 3));
+        reinterpret_cast<int4 *>(packed)[i] = w;
+        const uint32_t id = static_cast<uint32_t>(4 * i);
+        if (part) reinterpret_cast<uint4 *>(part)[i] = make_uint4(id, id + 1, id + 2, id + 3);
+        if (codes) reinterpret_cast<uchar4 *>(codes)[i] = make_uchar4(packed_code(w.x), packed_code(w.y), packed_code(w.z), packed_code(w.w));
+    }
+    if (blockIdx.x == 0 && threadIdx.x < n % 4) {
+        const uint64_t r = 4 * quads + threadIdx.x;
+        const int32_t w = quantize_row(spec, grad[r], hess[r], row_offset + r);
+        packed[r] = w;
+        if (part) part[r] = static_cast<uint32_t>(r);
+        if (codes) codes[r] = packed_code(w);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -2108,48 +2143,44 @@ __device__ __forceinline__ FeatCand categorical_candidate(const Ctx &c, const Sp
     return sorted_scan(c, cfg, m, u, sc, order_out);
 }
 
+// One feature's candidate from a leaf's histogram, by one wave: split.rs:584-620 find_numerical, or a categorical search.
+template <bool WIDE, class T>
+__device__ __forceinline__ FeatCand scan_feature(const Ctx &c, const SplitCfgDev &cfg, const FeatDev &m, const T *hist, bool evaluate,
+                                                 UnitPlanes<WIDE> &planes, CatScratch *cats, uint8_t *order_out) {
+    if (!scan_searched(c, m, evaluate)) return FeatCand{};
+    const auto u = stage_units<WIDE>(hist, m, planes);
+    Grown rg = {}, fg = {};
+    bool rf, ff;
+    if constexpr (WIDE) {
+        scan_numerical_wide(c, cfg, m, u, rf, rg, ff, fg);
+    } else {
+        if (m.kind == 2) return categorical_candidate(c, cfg, m, u, *cats, order_out);
+        scan_numerical(c, cfg, m, u, rf, rg, ff, fg);
+    }
+    return feature_candidate(c, m, rf, rg, ff, fg);
+}
+
 // split.rs:919-961 over one leaf's histogram, a wave a feature: split.rs:584-620 find_numerical, or a categorical search.
 // WIDE: the features of two-byte bins (numerical, up to 1024), in an instance of their own, so the wide scan's registers do
 // not lower the occupancy of the byte-bin scan. T: the histogram's units, int64_t, or double (a histogram of the host's,
 // read where the host put it). One wave a feature whatever its bins: all of a leaf's features are on the chip at once.
-// `from`, when set, holds the job (made on the device). grid: ceil(num_features / 4); 256 threads.
+// grid: ceil(num_features / 4); 256 threads.
 template <bool WIDE, class T>
-__global__ __launch_bounds__(256) void k_split_scan(ScanJob given, const ScanJob *from, const FeatDev *__restrict__ feats,
+__global__ __launch_bounds__(256) void k_split_scan(ScanJob job, const FeatDev *__restrict__ feats,
                                                     const uint8_t *__restrict__ evaluate, uint32_t num_features,
                                                     SplitCfgDev cfg, double sg, double sh,
-                                                    uint8_t *cat_order /* [feature][256] or null */,
-                                                    const DevScales *dsc /* when set: the scales */) {
+                                                    uint8_t *cat_order /* [feature][256] or null */) {
     __shared__ UnitPlanes<WIDE> planes[4];
     __shared__ __align__(16) uint8_t cats[WIDE ? 16 : 4 * sizeof(CatScratch)];
     const uint32_t wave = threadIdx.x >> 6, f = blockIdx.x * 4 + wave;
     if (f >= num_features) return;
     const FeatDev m = feats[f];
     const bool ev = evaluate[f] != 0;
-    const ScanJob job = from ? *from : given;
-    if (dsc) {
-        sg = dsc->sg;
-        sh = dsc->sh;
-    }
     if ((m.wide != 0) != WIDE) return;  // the other instance's feature
     const Ctx c = make_ctx(cfg, sg, sh, job.units_grad, job.units_hess, job.count);
-    FeatCand r = {};
-    if (scan_searched(c, m, ev)) {
-        const auto u = stage_units<WIDE>(reinterpret_cast<const T *>(job.hist), m, planes[wave]);
-        if constexpr (WIDE) {
-            Grown rg = {}, fg = {};
-            bool rf, ff;
-            scan_numerical_wide(c, cfg, m, u, rf, rg, ff, fg);
-            r = feature_candidate(c, m, rf, rg, ff, fg);
-        } else if (m.kind == 2) {
-            r = categorical_candidate(c, cfg, m, u, reinterpret_cast<CatScratch *>(cats)[wave],
-                                      cat_order ? cat_order + static_cast<size_t>(f) * 256 : nullptr);
-        } else {
-            Grown rg = {}, fg = {};
-            bool rf, ff;
-            scan_numerical(c, cfg, m, u, rf, rg, ff, fg);
-            r = feature_candidate(c, m, rf, rg, ff, fg);
-        }
-    }
+    const FeatCand r = scan_feature<WIDE>(c, cfg, m, reinterpret_cast<const T *>(job.hist), ev, planes[wave],
+                                          reinterpret_cast<CatScratch *>(cats) + (WIDE ? 0u : wave),
+                                          cat_order ? cat_order + static_cast<size_t>(f) * 256 : nullptr);
     if ((threadIdx.x & 63) == 0) job.out[f] = r;
 }
 
@@ -2506,7 +2537,6 @@ struct GrowState {
                               // slabs, then each two-byte feature's
     double *cand_gain;        // their gains (NaN as -inf) and features (-1: none), apart for coalesced loads
     int32_t *cand_feat;
-    uint8_t *evaluate;        // [nf]: the root's evaluated features
     const uint8_t *mask;      // [nf], the tree's feature mask
     const FeatDev *feats;
     TreeDev tree;
@@ -2607,86 +2637,92 @@ __global__ void k_copy_back(const MergeJob *__restrict__ jobs, const uint32_t *_
 }
 
 // The tree at its start: one leaf holding the root rows, its histogram in slot 0 when it is searched.
-__global__ void k_grow_init(GrowState g, uint32_t root_begin, uint32_t root_count, int64_t root_cnt, uint32_t searched) {
-    if (threadIdx.x == 0) {
-        GrowCtl &c = *g.ctl;
-        c.num_leaves = 1;
-        c.done = searched ? 0u : 1u;
-        c.error = 0;
-        c.ntent = 1;
-        c.next_slot = 1;
-        c.pending = 0;
-        c.steps = 0;
-        c.expansions = 0;
-        c.hist_rows = 0.0;
-        c.hist_bins = 0.0;
-        c.hist_builds = 0.0;
-        c.part_rows = 0.0;
-        TLeaf l = {};
-        l.begin = root_begin;
-        l.count = root_count;
-        l.cnt = root_cnt;
-        l.slot = searched ? 0 : -1;
-        l.state = T_LEAF;
-        l.kid = -1;
-        g.tl[0] = l;
-        g.tk[0] = TKey{0.0, 0u, T_LEAF, -1, 0u};
-        g.leaf_t[0] = 0;
-        g.leaf_left[0] = 0;
-        g.tree.leaf_value[0] = 0.0;
-        g.tree.leaf_weight[0] = 0.0;
-        g.tree.leaf_count[0] = 0;
-        g.tree.leaf_parent[0] = -1;
-        g.tree.leaf_depth[0] = 0;
-        g.tree.leaf_range[0] = root_begin;
-        g.tree.leaf_range[1] = root_count;
-        // both step plans empty until advance writes one: a step launched on an empty plan does nothing
-        for (int k = 0; k < 2; ++k) {
-            g.plans[k].njobs = 0;
-            g.plans[k].total_groups = 0;
-            g.plans[k].total_child = 0;
-            g.plans[k].total_red = 0;
-            g.plans[k].total_scan = 0;
-        }
+// A tree's state before its root is searched (or, `searched` 0, for a root that is not): by one thread.
+__device__ __forceinline__ void grow_init(const GrowState &g, uint32_t root_begin, uint32_t root_count, int64_t root_cnt,
+                                          uint32_t searched, double ug, double uh) {
+    GrowCtl &c = *g.ctl;
+    c.num_leaves = 1;
+    c.done = searched ? 0u : 1u;
+    c.error = 0;
+    c.ntent = 1;
+    c.next_slot = 1;
+    c.pending = 0;
+    c.steps = 0;
+    c.expansions = 0;
+    c.hist_rows = 0.0;
+    c.hist_bins = 0.0;
+    c.hist_builds = 0.0;
+    c.part_rows = 0.0;
+    TLeaf l = {};
+    l.begin = root_begin;
+    l.count = root_count;
+    l.ug = ug;
+    l.uh = uh;
+    l.cnt = root_cnt;
+    l.slot = searched ? 0 : -1;
+    l.state = T_LEAF;
+    l.kid = -1;
+    g.tl[0] = l;
+    g.tk[0] = TKey{0.0, 0u, T_LEAF, -1, 0u};
+    g.leaf_t[0] = 0;
+    g.leaf_left[0] = 0;
+    g.tree.leaf_value[0] = 0.0;
+    g.tree.leaf_weight[0] = 0.0;
+    g.tree.leaf_count[0] = 0;
+    g.tree.leaf_parent[0] = -1;
+    g.tree.leaf_depth[0] = 0;
+    g.tree.leaf_range[0] = root_begin;
+    g.tree.leaf_range[1] = root_count;
+    // both step plans empty until advance writes one: a step launched on an empty plan does nothing
+    for (int k = 0; k < 2; ++k) {
+        g.plans[k].njobs = 0;
+        g.plans[k].total_groups = 0;
+        g.plans[k].total_child = 0;
+        g.plans[k].total_red = 0;
+        g.plans[k].total_scan = 0;
     }
 }
+__global__ void k_grow_init(GrowState g, uint32_t root_begin, uint32_t root_count, int64_t root_cnt) {
+    if (threadIdx.x == 0) grow_init(g, root_begin, root_count, root_cnt, 0u, 0.0, 0.0);
+}
 
-// learner.rs:143-156: the root's sums from the sums feature's bins (split.rs:101-108), and its search job.
-// The root's sums are those of one feature's bins taken in bin order as f64. Every bin and every partial sum is an
-// integer of magnitude below 2^53 (rows times units stays below 2^48), so each of those additions is exact and the
-// result is the exact integer sum, which the block adds in i64 and converts once. grid: 1, 256 threads.
-__global__ __launch_bounds__(256) void k_root_prep(GrowState g) {
-    __shared__ int64_t part[2][4];
-    const TLeaf &l = g.tl[0];
-    const int64_t *h = g.pool + (size_t)l.slot * g.slot_stride;
-    for (uint32_t f = threadIdx.x; f < g.nf; f += blockDim.x) g.evaluate[f] = g.mask[f];
-    const FeatDev m = g.feats[g.sums_feature];
+// The root's search (learner.rs:143-157): its sums from the sums feature's bins (split.rs:101-108) and every feature's
+// candidate, a wave a feature; block 0 of the instance with `first` also makes the tree's initial state. The root's sums
+// are those of one feature's bins taken in bin order as f64; every bin and every partial sum is an integer of magnitude
+// below 2^53 (rows times units stays below 2^48), so each of those additions is exact and the result is the exact integer
+// sum, which every wave adds in i64 and converts once (one more round of loads, against the two launches this took
+// before). WIDE as k_split_scan's. grid: ceil(nf / 4), 256 threads.
+template <bool WIDE>
+__global__ __launch_bounds__(256) void k_root_scan(GrowState g, uint32_t root_begin, uint32_t root_count, int64_t root_cnt,
+                                                   uint32_t first) {
+    __shared__ UnitPlanes<WIDE> planes[4];
+    __shared__ __align__(16) uint8_t cats[WIDE ? 16 : 4 * sizeof(CatScratch)];
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u, f = blockIdx.x * 4 + wave;
+    const int64_t *hist = g.pool;  // the root's slot is 0
+    const FeatDev sums = g.feats[g.sums_feature];
+    const FeatDev m = f < g.nf ? g.feats[f] : FeatDev{};
+    const bool ev = f < g.nf && g.mask[f] != 0;
+    const double scale_g = grow_sg(g), scale_h = grow_sh(g);
+    const longlong2 *h = reinterpret_cast<const longlong2 *>(hist) + sums.hist_offset;
     int64_t sg = 0, sh = 0;
-    for (uint32_t b = threadIdx.x; b < m.num_bins; b += blockDim.x) {
-        sg += h[2 * ((size_t)m.hist_offset + b)];
-        sh += h[2 * ((size_t)m.hist_offset + b) + 1];
+    for (uint32_t b = lane; b < sums.num_bins; b += 64u) {
+        const longlong2 v = h[b];
+        sg += v.x;
+        sh += v.y;
     }
     for (int o = 32; o > 0; o >>= 1) {
         sg += static_cast<int64_t>(__shfl_xor(static_cast<long long>(sg), o));
         sh += static_cast<int64_t>(__shfl_xor(static_cast<long long>(sh), o));
     }
-    const uint32_t wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63u) == 0) {
-        part[0][wave] = sg;
-        part[1][wave] = sh;
+    const double dg = static_cast<double>(sg), dh = static_cast<double>(sh);
+    if (first && blockIdx.x == 0 && threadIdx.x == 0) {
+        grow_init(g, root_begin, root_count, root_cnt, 1u, dg, dh);
+        g.jobs[0] = ScanJob{hist, dg, dh, root_cnt, g.root_cands};
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int64_t tg = 0, th = 0;
-        for (uint32_t w = 0; w < blockDim.x / 64; ++w) {
-            tg += part[0][w];
-            th += part[1][w];
-        }
-        const double dg = static_cast<double>(tg), dh = static_cast<double>(th);
-        g.tl[0].ug = dg;
-        g.tl[0].uh = dh;
-        g.jobs[0] = ScanJob{h, dg, dh, l.cnt, g.root_cands};
-    }
+    if (f >= g.nf || (m.wide != 0) != WIDE) return;
+    const Ctx c = make_ctx(g.cfg, scale_g, scale_h, dg, dh, root_cnt);
+    const FeatCand r = scan_feature<WIDE>(c, g.cfg, m, hist, ev, planes[wave], reinterpret_cast<CatScratch *>(cats) + (WIDE ? 0u : wave), nullptr);
+    if (lane == 0) g.root_cands[f] = r;
 }
 
 // ---------------------------------------------------------------------------------------------------------
