@@ -269,6 +269,8 @@ struct HostTree {
 // ---------------------------------------------------------------------------------------------------------
 
 constexpr uint32_t RANK_DEVICE_MAX = 512;  // rows of the largest query k_rank_pairs takes (longer ones: the host's)
+constexpr int HIST_PART = 32;              // columns of a histogram workgroup that takes part of its rows' columns
+constexpr uint32_t HIST_PART_ROWS = 6144;  // rows a compute unit up to which histograms go by column parts (hist_parts)
 constexpr uint32_t HIST_MIN_ROWS = 2048;   // rows per histogram workgroup before another one is used
 constexpr uint64_t ROW_BLOCK = 256;
 
@@ -1383,6 +1385,21 @@ struct Context {
         return std::max<uint32_t>(1, std::min<uint32_t>(want, hist_cap));
     }
 
+    // The column parts of a byte slab's histogram workgroups (k_hist's SUB), 32 columns each, one workgroup a compute unit:
+    // up to HIST_PART_ROWS rows a unit, or where the partials' buffer holds no more row ranges than this takes. With whole
+    // rows a leaf of few rows leaves units idle or with a handful of dependent gathers, and a range's partial is written by
+    // one unit. Whole rows against parts, histogram and reduce, us: 128 columns 21k rows 20.6 / 10.4, 202k 26.9 / 15.3,
+    // 900k 43.3 / 34.2, 1.5M 64.8 / 62.9, 2M 89.4 / 91.6, 10M 309 / 407 (k_hist alone; a row's line is asked for four
+    // times); 64 columns 30k 14.3 / 9.9, 503k 23.3 / 19.2, 1.8M 38.6 / 33.8, 3.6M 69.4 / 72.4; 128 columns over the 64
+    // ranges of the fixed scratch: 202k 30.5 / 15.3, 2M 218 / 92. A part's i32 sums hold what `groups` ranges of whole rows
+    // hold, or 4 * HIST_PART_ROWS rows of at most 255 units (separate counters take the larger ones).
+    uint32_t hist_parts(const Slab &s, uint64_t count, uint32_t groups) const {
+        const int k = s.kernel();
+        if (k != 64 && k != 128) return 1u;
+        const uint32_t parts = static_cast<uint32_t>(k / HIST_PART);
+        return count <= static_cast<uint64_t>(HIST_PART_ROWS) * cus || groups * parts <= cus ? parts : 1u;
+    }
+
     // The histogram of rows part[begin..+count] (or the `side` child of that range split at *dev_left) into
     // `out` (i64 {g,h} per bin), and parent -= out when `parent` is set.
     // The features a histogram build evaluates: their columns, their bin bytes a row (two for a feature of
@@ -1411,7 +1428,8 @@ struct Context {
     void launch_hist_into(uint32_t begin, uint32_t count, const uint32_t *dev_left, uint32_t side, int64_t *out,
                           int64_t *parent, const HistUse &use, int32_t *partials, uint32_t grid, bool profiled) {
         for (auto &s : slabs) {
-            HistArgs a{slab_bins.p + s.bins_off, part.p, packed.p, partials, dev_left, begin, count, side, flush_rows(), grid, HIST_MIN_ROWS,
+            const uint32_t parts = hist_parts(s, count, grid), groups = parts > 1 ? std::min(grid, std::max(1u, cus / parts)) : grid;
+            HistArgs a{slab_bins.p + s.bins_off, part.p, packed.p, partials, dev_left, begin, count, side, flush_rows(), groups, HIST_MIN_ROWS,
                        slab_pos_word.p + s.pos_off, s.row_bytes() / 4};
             hipEvent_t e0 = nullptr, e1 = nullptr;
             if (profiled) {
@@ -1419,26 +1437,34 @@ struct Context {
                 e1 = event();
                 hip_check(hipEventRecord(e0, stream), "event");
             }
+            // the row ranges in eights (k_hist's order of the parts)
+            const uint32_t split = div_up(groups, 8) * 8 * parts;
             switch (s.kernel()) {
-            case 32: k_hist<32><<<grid, 1024, 0, stream>>>(a); break;
-            case 64: k_hist<64><<<grid, 1024, 0, stream>>>(a); break;
-            case 128: k_hist<128><<<grid, 1024, 0, stream>>>(a); break;
-            case 33: k_hist<32, true><<<grid, 1024, 0, stream>>>(a); break;
-            case 65: k_hist<64, true><<<grid, 1024, 0, stream>>>(a); break;
-            case 129: k_hist<128, true><<<grid, 1024, 0, stream>>>(a); break;
-            case 36: k_hist<32, false, 4><<<grid, 1024, 0, stream>>>(a); break;
-            case 68: k_hist<64, false, 4><<<grid, 1024, 0, stream>>>(a); break;
-            case 34: k_hist<32, false, 2><<<grid, 1024, 0, stream>>>(a); break;
-            case 66: k_hist<64, false, 2><<<grid, 1024, 0, stream>>>(a); break;
-            case 130: k_hist<128, false, 2><<<grid, 1024, 0, stream>>>(a); break;
-            case 3001: k_hist<128, false, 1, false, 1><<<grid, 1024, 0, stream>>>(a); break;
-            case 3002: k_hist<128, false, 1, false, 2><<<grid, 1024, 0, stream>>>(a); break;
-            case 3004: k_hist<128, false, 1, false, 4><<<grid, 1024, 0, stream>>>(a); break;
-            case 3008: k_hist<128, false, 1, false, 8><<<grid, 1024, 0, stream>>>(a); break;
-            case 1032: k_hist<32, false, 1, true><<<grid, 1024, 0, stream>>>(a); break;
-            case 1064: k_hist<64, false, 1, true><<<grid, 1024, 0, stream>>>(a); break;
-            case 1033: k_hist<32, true, 1, true><<<grid, 1024, 0, stream>>>(a); break;
-            case 1065: k_hist<64, true, 1, true><<<grid, 1024, 0, stream>>>(a); break;
+            case 32: k_hist<32><<<groups, 1024, 0, stream>>>(a); break;
+            case 64:
+                if (parts > 1) k_hist<64, false, 1, false, 0, HIST_PART><<<split, 1024, 0, stream>>>(a);
+                else k_hist<64><<<groups, 1024, 0, stream>>>(a);
+                break;
+            case 128:
+                if (parts > 1) k_hist<128, false, 1, false, 0, HIST_PART><<<split, 1024, 0, stream>>>(a);
+                else k_hist<128><<<groups, 1024, 0, stream>>>(a);
+                break;
+            case 33: k_hist<32, true><<<groups, 1024, 0, stream>>>(a); break;
+            case 65: k_hist<64, true><<<groups, 1024, 0, stream>>>(a); break;
+            case 129: k_hist<128, true><<<groups, 1024, 0, stream>>>(a); break;
+            case 36: k_hist<32, false, 4><<<groups, 1024, 0, stream>>>(a); break;
+            case 68: k_hist<64, false, 4><<<groups, 1024, 0, stream>>>(a); break;
+            case 34: k_hist<32, false, 2><<<groups, 1024, 0, stream>>>(a); break;
+            case 66: k_hist<64, false, 2><<<groups, 1024, 0, stream>>>(a); break;
+            case 130: k_hist<128, false, 2><<<groups, 1024, 0, stream>>>(a); break;
+            case 3001: k_hist<128, false, 1, false, 1><<<groups, 1024, 0, stream>>>(a); break;
+            case 3002: k_hist<128, false, 1, false, 2><<<groups, 1024, 0, stream>>>(a); break;
+            case 3004: k_hist<128, false, 1, false, 4><<<groups, 1024, 0, stream>>>(a); break;
+            case 3008: k_hist<128, false, 1, false, 8><<<groups, 1024, 0, stream>>>(a); break;
+            case 1032: k_hist<32, false, 1, true><<<groups, 1024, 0, stream>>>(a); break;
+            case 1064: k_hist<64, false, 1, true><<<groups, 1024, 0, stream>>>(a); break;
+            case 1033: k_hist<32, true, 1, true><<<groups, 1024, 0, stream>>>(a); break;
+            case 1065: k_hist<64, true, 1, true><<<groups, 1024, 0, stream>>>(a); break;
             default: throw std::logic_error("no histogram kernel for the slab");
             }
             launch_check("k_hist");
@@ -1447,8 +1473,8 @@ struct Context {
                 prof.hist_events.emplace_back(e0, e1);
                 prof.hist_launches += 1;
             }
-            ReduceArgs r{partials, s.col_offset.p, s.col_bins.p, s.col_stride.p, out, parent, dev_left, begin, count, side, grid, HIST_MIN_ROWS, s.width, s.seg_shift(),
-                         s.dense_passes ? slab_slot_flat.p + s.slot_off : nullptr};
+            ReduceArgs r{partials, s.col_offset.p, s.col_bins.p, s.col_stride.p, out, parent, dev_left, begin, count, side, groups, HIST_MIN_ROWS, q32 ? 0u : flush_rows(),
+                         s.width, s.seg_shift(), s.dense_passes ? slab_slot_flat.p + s.slot_off : nullptr};
             k_hist_reduce<<<div_up(256ull * s.width, 32), 256, 0, stream>>>(r);
             launch_check("k_hist_reduce");
         }

@@ -329,18 +329,19 @@ __global__ void k_iota(uint32_t *__restrict__ out, uint64_t n) {
 // Every `flush_rows` rows (at most 32767 / max |g| and 65535 / max h: the low half holds g as a signed 16-bit
 // value, the high half h, which is never negative, as an unsigned one) the packed words are unpacked into per-thread
 // registers (i32 g and h sums) and zeroed. Each workgroup writes its sums as a partial
-// histogram `partial[wg][bin * W + column] = {g, h}`; k_hist_reduce adds the partials.
+// histogram `partial[wg][bin * W + column] = {g, h}`, or, when its rows never need a flush, the packed words themselves (half
+// the bytes: 128 columns, 202k rows over 98 workgroups 32.0 -> 26.7 us with the reduce); k_hist_reduce adds the partials.
 // ---------------------------------------------------------------------------------------------------------
 
 struct HistArgs {
     const uint8_t *bins;      // slab rows: row r at bins + r * W
     const uint32_t *rows;     // partition buffer; the leaf's rows start at `begin`
     const int32_t *gh;        // packed quantized gradients per row
-    int32_t *partial;         // [grid][256 * W][2]
+    int32_t *partial;         // [groups][256 * W] {g, h} pairs, or packed words in the first half of each
     const uint32_t *dev_left; // when non-null: the leaf is the `side` child of [begin, begin+count) split at *dev_left
     uint32_t begin, count, side;
     uint32_t flush_rows;
-    uint32_t max_groups;      // == gridDim.x
+    uint32_t max_groups;      // row ranges at most
     uint32_t min_rows_per_group;
     const uint32_t *pos_word; // dense slab: per row byte, its LDS word at bin 0 (segment base * W + column)
     uint32_t dw_row;          // dense slab: dwords per row
@@ -503,26 +504,34 @@ __device__ __forceinline__ void hist_list_dense(int32_t *lds, const uint32_t *li
 // zeroed, so the compiler issues every load of a step back to back instead of one masked load at a time. A
 // wave fetches the row ids of its next step in one coalesced load (lane l: id l) while it works on the current
 // step, and hands them out with a shuffle. WIDE: the slab's rows are W / 4 two-byte bins. PACK: the slab's rows
-// are W * PACK bytes, PACK features of at most 256 / PACK bins to an LDS column.
-template <int W, bool WIDE = false, int PACK = 1, bool Q32 = false, int DP = 0>
+// are W * PACK bytes, PACK features of at most 256 / PACK bins to an LDS column. SUB: the columns a workgroup takes of its
+// rows; W / SUB workgroups share a row range, each reading its dwords of every row.
+template <int W, bool WIDE = false, int PACK = 1, bool Q32 = false, int DP = 0, int SUB = W>
 __global__ __launch_bounds__(1024) void k_hist(HistArgs a) {
     static_assert(PACK == 1 || (!WIDE && W * PACK <= 256), "a packed row is at most 64 dwords");
     static_assert(!Q32 || W <= 64, "separate g and h counters take twice the LDS");
     static_assert(DP == 0 || (W == 128 && !WIDE && PACK == 1 && !Q32), "a dense slab has 128 byte columns");
-    constexpr int DW = WIDE ? W / 8 : W * PACK / 4;  // dwords per row
+    static_assert(SUB == W || (!WIDE && PACK == 1 && !Q32 && DP == 0), "only byte slabs go by column parts");
+    constexpr int PARTS = W / SUB;                      // workgroups that share a row range, each with SUB of the columns
+    constexpr int ROW = WIDE ? W / 8 : W * PACK / 4;    // dwords per row
+    constexpr int DW = ROW / PARTS;                     // of them, this workgroup's
     constexpr int RPW = WAVE / DW;            // rows per wave step
     // row ids of one step fit one wave-wide load; at W = 128 the 64 accumulator registers leave room for 8
-    constexpr int UNROLL = W == 128 ? 8 : (64 / RPW < 16 ? 64 / RPW : 16);
+    constexpr int UNROLL = SUB == 128 ? 8 : (64 / RPW < 16 ? 64 / RPW : 16);
     constexpr uint32_t STEP = 16u * RPW * UNROLL;          // rows per block step (16 waves)
-    constexpr int SLOTS = 256 * W / 1024;
-    constexpr int LDS_WORDS = (Q32 ? 2 : 1) * 256 * W + (DP ? W : 0);  // a dense slab's spare row
+    constexpr int SLOTS = 256 * SUB / 1024;
+    constexpr int LDS_WORDS = (Q32 ? 2 : 1) * 256 * SUB + (DP ? W : 0);  // a dense slab's spare row
     __shared__ int32_t lds[LDS_WORDS];
 
     uint32_t lb, n;
     leaf_rows(a.dev_left, a.begin, a.count, a.side, lb, n);
     uint32_t groups, per;
     hist_split(n, a.max_groups, a.min_rows_per_group, groups, per);
-    if (blockIdx.x >= groups) return;
+    // the parts of a row range 8 workgroups apart, so on one XCD: its L2 serves a row's line to all but the first
+    const uint32_t group = PARTS == 1 ? blockIdx.x : blockIdx.x / (8u * PARTS) * 8u + blockIdx.x % 8u;
+    const uint32_t part = PARTS == 1 ? 0u : blockIdx.x / 8u % PARTS;
+    if (group >= groups) return;
+    const bool packed = !Q32 && per <= a.flush_rows;  // the partial is the packed words themselves
     const uint32_t tid = threadIdx.x;
     for (uint32_t k = tid; k < static_cast<uint32_t>(LDS_WORDS); k += 1024) lds[k] = 0;
     int32_t accg[SLOTS], acch[SLOTS];
@@ -534,10 +543,10 @@ __global__ __launch_bounds__(1024) void k_hist(HistArgs a) {
     const uint32_t d = lane % DW, rsub = lane / DW;
     const uint32_t rot = (lane & 31u) >> 3;
     uint32_t xs[4], cols[4];
-    row_bin_lanes<W, PACK>(d, rot, xs, cols);
+    row_bin_lanes<SUB, PACK>(d, rot, xs, cols);
     const uint32_t *rows = a.rows + lb;
-    const uint32_t *bins32 = reinterpret_cast<const uint32_t *>(a.bins);
-    uint32_t start = blockIdx.x * per;
+    const uint32_t *bins32 = reinterpret_cast<const uint32_t *>(a.bins) + part * DW;
+    uint32_t start = group * per;
     uint32_t end = start + per < n ? start + per : n;
     uint32_t dcols[DP ? DP : 1][4];
     if constexpr (DP > 0) dense_lanes<DP>(a.pos_word, lane, xs, dcols);
@@ -560,18 +569,19 @@ __global__ __launch_bounds__(1024) void k_hist(HistArgs a) {
 #pragma unroll
                 for (int u = 0; u < UNROLL; ++u) {
                     g[u] = a.gh[r[u]];
-                    dw[u] = bins32[(size_t)r[u] * DW + d];
+                    dw[u] = bins32[(size_t)r[u] * ROW + d];
                 }
 #pragma unroll
                 for (int u = 0; u < UNROLL; ++u) {
                     int32_t gv, hv;
                     row_units<Q32>(g[u], base + u * RPW + rsub < cend, gv, hv);
                     if constexpr (WIDE) add_row_bins_wide<W, Q32>(lds, dw[u], gv, hv, d);
-                    else add_row_bins<W, PACK, Q32>(lds, dw[u], gv, hv, xs, cols);
+                    else add_row_bins<SUB, PACK, Q32>(lds, dw[u], gv, hv, xs, cols);
                 }
             }
         }
         __syncthreads();
+        if (packed) break;  // the only chunk
 #pragma unroll
         for (int j = 0; j < SLOTS; ++j) {
             int32_t v = lds[tid + j * 1024];
@@ -588,9 +598,22 @@ __global__ __launch_bounds__(1024) void k_hist(HistArgs a) {
         }
         __syncthreads();
     }
-    int2 *out = reinterpret_cast<int2 *>(a.partial) + (size_t)blockIdx.x * (256 * W);
+    // the slot of LDS word k: bin k / SUB, column part * SUB + k % SUB
+    int32_t *mine = a.partial + static_cast<size_t>(group) * (2 * 256 * W);
+    if (packed) {
 #pragma unroll
-    for (int j = 0; j < SLOTS; ++j) out[tid + j * 1024] = make_int2(accg[j], acch[j]);
+        for (int j = 0; j < SLOTS; ++j) {
+            const uint32_t k = tid + j * 1024;
+            mine[k / SUB * W + part * SUB + k % SUB] = lds[k];
+        }
+        return;
+    }
+    int2 *out = reinterpret_cast<int2 *>(mine);
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j) {
+        const uint32_t k = tid + j * 1024;
+        out[k / SUB * W + part * SUB + k % SUB] = make_int2(accg[j], acch[j]);
+    }
 }
 
 // Adds the partials of one slab into the leaf histogram (i64 {g, h} per bin, flat layout). Thread per slab slot
@@ -607,6 +630,7 @@ struct ReduceArgs {
     const uint32_t *dev_left;
     uint32_t begin, count, side;
     uint32_t max_groups, min_rows_per_group;
+    uint32_t packed_rows; // partials of at most this many rows are packed words (k_hist)
     uint32_t width;     // W
     uint32_t seg_shift; // a packed slab's column holds a feature each 2^seg_shift bins: 8 (one feature), 7 or 6
     const uint32_t *slot_flat;  // a dense slab: per slot (bin * W + column) its flat-histogram bin + 1, 0 for none
@@ -630,12 +654,22 @@ __global__ __launch_bounds__(256) void k_hist_reduce(ReduceArgs a) {
     const bool on = s < slots && (a.slot_flat ? flat1 != 0u : vb < a.col_bins[fs]);
     int64_t g = 0, h = 0;
     if (on) {
-        const int2 *p = reinterpret_cast<const int2 *>(a.partial) + s;
+        if (per <= a.packed_rows) {
+            const int32_t *p = a.partial + s;
 #pragma unroll 8
-        for (uint32_t w = stripe; w < groups; w += 8u) {
-            const int2 v = p[static_cast<size_t>(w) * slots];
-            g += v.x;
-            h += v.y;
+            for (uint32_t w = stripe; w < groups; w += 8u) {
+                const int32_t v = p[2 * static_cast<size_t>(w) * slots], gq = packed_g(v);
+                g += gq;
+                h += packed_h(v, gq);
+            }
+        } else {
+            const int2 *p = reinterpret_cast<const int2 *>(a.partial) + s;
+#pragma unroll 8
+            for (uint32_t w = stripe; w < groups; w += 8u) {
+                const int2 v = p[static_cast<size_t>(w) * slots];
+                g += v.x;
+                h += v.y;
+            }
         }
     }
     red[0][stripe][lane] = g;
