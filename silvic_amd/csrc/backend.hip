@@ -436,7 +436,7 @@ struct Context {
     Pinned<float> h_lv;
     DevBuf<uint16_t> leaf_of;  // each training row's leaf in the last tree (k_tree_leaves)
     DevBuf<float> d_leaf_values;
-    DevBuf<LeafJob> d_leaf_jobs;
+    DevBuf<unsigned long long> d_leaf_jobs;     // leaf_sums: its sums, then its jobs
     DevBuf<unsigned long long> d_leaf_out;
 
     srocm_rank::Ranker ranker;  // lambdarank: the setup, the sigmoid and discount tables
@@ -1651,23 +1651,27 @@ struct Context {
         for (uint32_t i = 0; i < n; ++i) check_range(leaves[i]);
         ensure_order();
         if (n == 0) return;
-        std::vector<LeafJob> jobs(n);
-        uint32_t maxc = 0;
-        for (uint32_t i = 0; i < n; ++i) {
-            jobs[i] = LeafJob{leaves[i].begin, leaves[i].count, i};
-            maxc = std::max(maxc, leaves[i].count);
+        // the zeroed sums and the jobs after them, in one copy
+        size_t njobs = 0;
+        for (uint32_t i = 0; i < n; ++i) njobs += div_up(leaves[i].count, LEAF_SUM_ROWS);
+        const size_t words = 2 * static_cast<size_t>(n) + div_up(njobs * sizeof(LeafJob), 8);
+        Pinned<unsigned long long> &h = h_sums;  // the upload's staging, then the readback's
+        h.alloc(words);
+        d_leaf_jobs.alloc(words);
+        std::fill(h.p, h.p + 2 * static_cast<size_t>(n), 0ull);
+        auto *jobs = reinterpret_cast<LeafJob *>(h.p + 2 * static_cast<size_t>(n));
+        for (uint32_t i = 0; i < n; ++i)
+            for (uint64_t at = 0; at < leaves[i].count; at += LEAF_SUM_ROWS)
+                *jobs++ = LeafJob{leaves[i].begin + static_cast<uint32_t>(at),
+                                  static_cast<uint32_t>(std::min<uint64_t>(leaves[i].count - at, LEAF_SUM_ROWS)), i};
+        hip_check(hipMemcpyAsync(d_leaf_jobs.p, h.p, words * 8, hipMemcpyHostToDevice, stream), "upload leaves");
+        if (njobs) {
+            k_leaf_sums<<<static_cast<uint32_t>(njobs), 256, 0, stream>>>(grad.p, hess.p, part.p,
+                                                                          reinterpret_cast<const LeafJob *>(d_leaf_jobs.p + 2 * static_cast<size_t>(n)),
+                                                                          gs, hs, d_leaf_jobs.p);
+            launch_check("k_leaf_sums");
         }
-        d_leaf_jobs.alloc(n);
-        d_leaf_out.alloc(2 * n);
-        hip_check(hipMemcpyAsync(d_leaf_jobs.p, jobs.data(), n * sizeof(LeafJob), hipMemcpyHostToDevice, stream), "upload leaves");
-        hip_check(hipMemsetAsync(d_leaf_out.p, 0, 2 * n * 8, stream), "zero sums");
-        uint32_t chunk = 8192;
-        dim3 grid(std::max<uint32_t>(1, div_up(maxc, chunk)), n);
-        k_leaf_sums<<<grid, 256, 0, stream>>>(grad.p, hess.p, part.p, d_leaf_jobs.p, gs, hs, d_leaf_out.p, chunk);
-        launch_check("k_leaf_sums");
-        Pinned<unsigned long long> &h = h_sums;
-        h.alloc(2 * n);
-        hip_check(hipMemcpyAsync(h.p, d_leaf_out.p, 2 * n * 8, hipMemcpyDeviceToHost, stream), "read sums");
+        hip_check(hipMemcpyAsync(h.p, d_leaf_jobs.p, 2 * n * 8, hipMemcpyDeviceToHost, stream), "read sums");
         sync();
         for (uint32_t i = 0; i < 2 * n; ++i) out[i] = static_cast<int64_t>(h.p[i]);
     }
@@ -1709,8 +1713,32 @@ struct Context {
         if (d.rows == 0) return;
         if (nn == 0) k_add_const<<<grid_rows(d.rows), 256, 0, stream>>>(d.scores.p, d.rows, v0);
         else if (from_leaf_of) k_add_leaf_values<<<grid_rows(d.rows), 256, 0, stream>>>(leaf_of.p, d_leaf_values.p, d.scores.p, d.rows, nullptr);
-        else k_add_tree<<<grid_rows(d.rows), 256, 0, stream>>>(d.col.p, col16, d.rows, d_nodes.p, d_leaf_values.p, d.scores.p, nullptr);
+        else launch_add_tree(d, nn + 1, nullptr);
         launch_check("k_add_tree");
+    }
+
+    template <bool COL16>
+    void launch_add_tree_walk(DevData &d, uint32_t nl, const uint32_t *gate) {
+        constexpr uint32_t threads = tl_threads<LEAVES_SMALL>();
+        static const int per_cu = [] {
+            int n = 0;
+            hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_add_tree_walk<COL16>, threads, 0), "occupancy");
+            return n > 0 ? n : 1;
+        }();
+        const uint32_t grid = static_cast<uint32_t>(std::min<uint64_t>(static_cast<uint64_t>(per_cu) * cus,
+                                                                        div_up(d.rows, static_cast<uint64_t>(tl_rows<LEAVES_SMALL>()) * threads)));
+        k_add_tree_walk<COL16><<<grid, threads, 0, stream>>>(d.col.p, static_cast<uint32_t>(d.rows), d_nodes.p, nl, d_leaf_values.p, d.scores.p, gate);
+    }
+
+    // scores += the leaf values of the tree in d_nodes, of at most nl leaves (the gate, when set, holds the actual count).
+    // Below 1024 rows a compute unit the staging of the nodes costs more than it saves (k_add_tree against the walk: 60k
+    // rows 8.6 / 10.4 us, 300k 10.8 / 10.8, 1M 37.9 / 17.6), and with more than 512 leaves at every size (staged in blocks of
+    // 1024 threads, 1000 leaves: 9k rows 16.6 / 72 us, 2M 94 / 121).
+    void launch_add_tree(DevData &d, uint32_t nl, const uint32_t *gate) {
+        if (d.rows < 1024ull * cus || d.rows >> 32 || nl > LEAVES_SMALL)
+            k_add_tree<<<grid_rows(d.rows), 256, 0, stream>>>(d.col.p, col16, d.rows, d_nodes.p, d_leaf_values.p, d.scores.p, gate);
+        else if (col16) launch_add_tree_walk<true>(d, nl, gate);
+        else launch_add_tree_walk<false>(d, nl, gate);
     }
 
     void add_tree(const srocm_device_node *nodes, uint32_t nn, const float *lv, uint32_t nl) {
@@ -2881,7 +2909,7 @@ uint32_t Context::boost(const srocm_train_params &p, uint32_t first, uint32_t co
             if (train.rows)
                 k_add_leaf_values<<<grid_rows(train.rows), 256, 0, stream>>>(leaf_of.p, d_leaf_values.p, train.scores.p, train.rows, d_gate.p);
             for (auto &v : valid)
-                if (v.rows) k_add_tree<<<grid_rows(v.rows), 256, 0, stream>>>(v.col.p, col16, v.rows, d_nodes.p, d_leaf_values.p, v.scores.p, d_gate.p);
+                if (v.rows) launch_add_tree(v, p.num_leaves, d_gate.p);
             launch_check("k_add_tree");
         };
         struct ScalesFromDevice {  // GrowState takes the device's scales while this tree grows
