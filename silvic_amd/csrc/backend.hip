@@ -1059,11 +1059,10 @@ struct Context {
                         held[col / CG_COLS].emplace_back(nt_feat[i], 256u * (col % CG_COLS) + row);
                     }
                 for (uint32_t c0 = 0; c0 < s.width; c0 += CG_COLS) {
-                    ColGroup x{poff, s.width, c0, static_cast<uint32_t>(si) * k1_groups(), {}, {}, {}, s.seg_shift(),
+                    ColGroup x{poff, s.width, c0, static_cast<uint32_t>(si) * k1_groups(), {}, {}, s.seg_shift(),
                                s.dense_passes ? 1u : 0u, static_cast<uint32_t>(s.slot_off), s.q32 ? 1u : 0u, 0u, 0u};
                     for (uint32_t k = 0; k < CG_COLS && !s.dense_passes; ++k) {
                         const uint32_t v = c0 + k;
-                        x.stride[k] = s.wide ? 4u : 1u;
                         for (uint32_t seg = 0; seg < s.pack; ++seg) {
                             const uint32_t c = s.wide ? v % cap : seg * s.width + v, q = s.wide ? v / cap : 0u;
                             const bool real = c < s.feats.size();

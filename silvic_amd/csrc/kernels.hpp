@@ -4762,7 +4762,6 @@ struct ColGroup {
     uint32_t fmt;      // the slab's first k_step_rows workgroup in the partial-format flags
     uint32_t offset[4][4];  // per segment and column: its feature's first bin in the flat histogram
     uint32_t bins[4][4];    // per segment and column: the feature's bins (0 for padding)
-    uint32_t stride[4];     // per column: flat-histogram bins between its consecutive bins (4 in a wide slab)
     uint32_t seg_shift;     // a column holds a feature each 2^seg_shift bins (8: one; 7 or 6 in a packed slab)
     uint32_t dense;         // a dense slab: the slots' flat bins come from the slot table at slot_base
     uint32_t slot_base;
@@ -5111,7 +5110,10 @@ __global__ __launch_bounds__(512, 4) void k_step_children(GrowState g, ChildArgs
 // subtraction in place of the parent's (learner.rs:356-371). Work items (job, column group, bin range) in a grid-stride
 // loop: a thread adds one stripe of the workgroups' partials of one bin of the group's four columns, reading each partial
 // in its own format (packed: one 16-byte load; {g, h} pairs: two), and the stripes meet in LDS. (A two-byte feature's
-// bins lie in four column groups, so its scan is a launch of its own.) grid: any, 256 threads.
+// bins lie in four column groups, so its scan is a launch of its own.) An item takes neighbouring bins of four features
+// across their four column groups, so that a wave reads and writes whole lines of the histograms: by column group a lane's
+// bins were 64 bytes from the next one's and each line was written by four items (6M x 32 at 2047 leaves 56 -> 38 us a
+// step). grid: any, 256 threads.
 __global__ __launch_bounds__(256) void k_step_reduce(GrowState g, ReduceStepArgs a) {
     __shared__ int64_t red[8][256];  // the stripes' sums, [value][thread]: conflict-free
     const StepPlan &P = *a.plan;  // empty once the tree is done (k_step_select)
@@ -5132,35 +5134,32 @@ __global__ __launch_bounds__(256) void k_step_reduce(GrowState g, ReduceStepArgs
             cgi = r / ways;
             sub = r - cgi * ways;
         }
-        const ColGroup &cg = a.cgs[cgi];  // read in place: a column is picked per thread
+        const ColGroup &cg = a.cgs[cgi];
         int64_t *built = g.pool + static_cast<size_t>(J.built_slot) * g.slot_stride;
         int64_t *parent = g.pool + static_cast<size_t>(J.parent_slot) * g.slot_stride;
         const size_t stride4 = step_partial_stride(cg.width) / 2;  // int4s from one partial to the next
         const uint32_t ns = 256u / ways;                           // the item's bins
         const uint32_t q = tid / ns;                               // this thread's stripe
-        const uint32_t bin = sub * ns + tid % ns;
+        // the slab's column group l stands for four features (quad) and a quarter of their 1024 bins; bin b lies in the
+        // column group of its phase b % 4, as bin b / 4 of the group's columns
+        const uint32_t l = cg.c0 / CG_COLS, nq = cg.width / (4u * CG_COLS), quad = l % nq;
+        const uint32_t b = (l / nq * ways + sub) * ns + tid % ns, bin = b / 4u, lb = (b % 4u) * nq + quad;
+        const ColGroup &cb = a.cgs[cgi - l + lb];
         // bin `bin` of the group's columns in a partial: int4 (bin / 4) * W + c0 + bin % 4, of packed words or, in a
         // partial of pairs, of its g plane, the h plane's 64 W int4s on
         const int4 *src = reinterpret_cast<const int4 *>(a.partial + 2 * cg.partial) + static_cast<size_t>(J.group_base) * stride4 +
-                          static_cast<size_t>(bin / 4u) * cg.width + cg.c0 + bin % 4u;
+                          static_cast<size_t>(bin / 4u) * cg.width + CG_COLS * lb + bin % 4u;
         const size_t plane = 64u * static_cast<size_t>(cg.width);
         const uint32_t *fmt = a.fmt + cg.fmt + J.group_base;
-        // the parent's bins are loaded with the partials (the writes below need them); every partial is first read
-        // as packed, and a {g, h} pair partial (a workgroup that flushed) is read again in its own layout
-        // the flat bin + 1 of each of the four columns' slot (0: none)
+        // the parent's bins are loaded with the partials (the writes below need them); fl: the flat bin + 1 of each of the
+        // four features' bin b (0: none)
         uint32_t fl[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) fl[c] = bin < cg.bins[0][c] ? cg.offset[0][c] + bin * cg.stride[c] + 1u : 0u;
-        int64_t pg[4] = {0, 0, 0, 0}, ph[4] = {0, 0, 0, 0};
+        for (int c = 0; c < 4; ++c) fl[c] = bin < cb.bins[0][c] ? cb.offset[0][c] + bin * 4u + 1u : 0u;
+        longlong2 par[4];
         if (q == 0) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                if (fl[c]) {
-                    const size_t o = 2 * static_cast<size_t>(fl[c] - 1u);
-                    pg[c] = parent[o];
-                    ph[c] = parent[o + 1];
-                }
-            }
+            for (int c = 0; c < 4; ++c) par[c] = *reinterpret_cast<const longlong2 *>(parent + 2 * static_cast<size_t>(fl[c] ? fl[c] - 1u : 0u));
         }
         int64_t sg[4] = {0, 0, 0, 0}, sh[4] = {0, 0, 0, 0};
         for (uint32_t w = q; w < groups; w += 8u * ways) {
@@ -5189,10 +5188,8 @@ __global__ __launch_bounds__(256) void k_step_reduce(GrowState g, ReduceStepArgs
             for (int c = 0; c < 4; ++c) {
                 if (fl[c]) {
                     const size_t o = 2 * static_cast<size_t>(fl[c] - 1u);
-                    built[o] = sg[c];
-                    built[o + 1] = sh[c];
-                    parent[o] = pg[c] - sg[c];
-                    parent[o + 1] = ph[c] - sh[c];
+                    *reinterpret_cast<longlong2 *>(built + o) = make_longlong2(sg[c], sh[c]);
+                    *reinterpret_cast<longlong2 *>(parent + o) = make_longlong2(par[c].x - sg[c], par[c].y - sh[c]);
                 }
             }
         }
